@@ -247,6 +247,23 @@ int run_operator(hd_advection *op, int mode, int precision, const void *src,
                   static_cast<float *>(dst), op->coef32, mf->mesh, op->inflow,
                   op->quad, stage, time, mf->dim_x, stream);
     }
+  else if (op->has_curved && op->algorithm == HD_ALGO_AUTO &&
+           (reinterpret_cast<uintptr_t>(src) |
+            reinterpret_cast<uintptr_t>(dst)) %
+               16 ==
+             0)
+    // a deformed mesh without boundaries: the factorised form of the
+    // quadrature operator (16-byte accesses; other vectors take the
+    // quadrature kernel, which HD_ALGO_QUADRATURE selects as well)
+    e = precision == HD_FP64
+          ? hd::curved_apply_f64(mf->dim_x, mf->dim_v, mf->nd, mode,
+                                 static_cast<const double *>(src),
+                                 static_cast<double *>(dst), op->curved,
+                                 mf->mesh, stage, stream)
+          : hd::curved_apply_f32(mf->dim_x, mf->dim_v, mf->nd, mode,
+                                 static_cast<const float *>(src),
+                                 static_cast<float *>(dst), op->curved,
+                                 mf->mesh, stage, stream);
   else if (precision == HD_FP64)
     e = hd::quadrature_apply(mf->D, mf->nd, mf->nq, mode,
                              static_cast<const double *>(src),
@@ -623,6 +640,22 @@ int hd_advection_create(hd_matrix_free *mf, const double *velocity,
       op->geo.xfg = parts[1];
       op->geo.vca = parts[2];
       op->geo.vfg = parts[3];
+      if (all_periodic && hd::curved_supported(mf->dim_x, mf->dim_v, nd,
+                                               mf->xmap.n_cells(),
+                                               mf->vmap.n_cells()))
+        {
+          hd::CurvedHost hx, hv;
+          hd::curved_space_operator(mf->xmap, t, skew_factor, xc, xf, hx);
+          hd::curved_space_operator(mf->vmap, t, skew_factor, vc, vf, hv);
+          e = hd::curved_create(mf->dim_x, mf->dim_v, nd, hx, hv,
+                                &op->curved);
+          if (e != hipSuccess)
+            {
+              hd_advection_destroy(op);
+              return hip_fail(e, "hd_advection_create: cell matrices");
+            }
+          op->has_curved = true;
+        }
     }
   mf->n_ops += 1;
   op->counted = true;
@@ -644,6 +677,7 @@ int hd_advection_destroy(hd_advection *op)
   if (op->mf && op->mf->n_ops > 0 && op->counted)
     op->mf->n_ops -= 1;
   hd_abi::learned_release(op->learned);
+  hd::curved_destroy(op->curved);
   if (op->fdm)
     {
       hd::vp_fdm_destroy(*op->fdm);

@@ -325,6 +325,30 @@ hipError_t quadrature_apply_f32(int D, int ND, int NQ, int mode,
                                 int dim_x, int collocation,
                                 const double *efield, const DeformDev &geo,
                                 hipStream_t stream);
+// Periodic deformed meshes with constant velocity in the factorised form
+// (hd_curved.hip): the per-cell matrices of the two spaces on the device
+// (lane order, FP64 and FP32) and, per cell, the face steps with inflow
+struct CurvedDev
+{
+  double *xtab64 = nullptr, *vtab64 = nullptr;
+  float *xtab32 = nullptr, *vtab32 = nullptr;
+  unsigned *xmask = nullptr, *vmask = nullptr;
+};
+struct CurvedHost;
+bool curved_supported(int dim_x, int dim_v, int N, long long n_x_cells,
+                      long long n_v_cells);
+hipError_t curved_create(int dim_x, int dim_v, int N, const CurvedHost &x,
+                         const CurvedHost &v, CurvedDev *out);
+void curved_destroy(CurvedDev &c);
+// src, dst 16-byte aligned
+hipError_t curved_apply_f64(int dim_x, int dim_v, int N, int mode,
+                            const double *src, double *dst,
+                            const CurvedDev &cv, const MeshDev &mesh,
+                            const StageDev &stage, hipStream_t stream);
+hipError_t curved_apply_f32(int dim_x, int dim_v, int N, int mode,
+                            const float *src, float *dst, const CurvedDev &cv,
+                            const MeshDev &mesh, const StageDev &stage,
+                            hipStream_t stream);
 // the face-centric form (MatrixFree::loop + the inverse-mass cell_loop):
 // cell, face (per direction and colour) and inverse-mass kernels; asmv is
 // the vector the integrals are assembled in (dst for an apply, ti_out or a

@@ -1,7 +1,9 @@
 // hd_geometry.cpp -- host-side geometry of a deformed phase-space mesh (see
 // hd_geometry.h).
 #include "hd_geometry.h"
+#include "hd_tables.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace hd
@@ -156,6 +158,129 @@ void space_tables(const SpaceMap &m, int nq, const double *xq,
               face[(((size_t)c * 2 * dim) + 2 * d + s) * nfpt + p] =
                 (s ? 1.0 : -1.0) * v * std::fabs(det) * w;
             }
+    }
+}
+
+void curved_space_operator(const SpaceMap &m, const Tables1D &t, double skew,
+                           const std::vector<double> &cell,
+                           const std::vector<double> &face, CurvedHost &out)
+{
+  const int dim = m.dim, nd = t.nd, nq = t.nq;
+  int n = 1, np = 1, nf = 1, npf = 1;
+  for (int d = 0; d < dim; ++d)
+    {
+      n *= nd;
+      np *= nq;
+      if (d > 0)
+        {
+          nf *= nd;
+          npf *= nq;
+        }
+    }
+  const int sides = 2 * dim, nb = sides * nf;
+  out.cells = m.n_cells();
+  out.K.assign((size_t)out.cells * n * n, 0.0);
+  out.B.assign((size_t)out.cells * n * nb, 0.0);
+  // tensor products of the 1D tables: nodes -> points of the cell and of a
+  // face, points -> nodes
+  auto tensor = [](const std::vector<double> &A, int rows, int cols, int k) {
+    int R = 1, C = 1;
+    std::vector<double> r(1, 1.0);
+    for (int d = 0; d < k; ++d)
+      {
+        // direction d is slower than the ones before it
+        std::vector<double> s((size_t)R * rows * C * cols);
+        for (int i = 0; i < rows; ++i)
+          for (int a = 0; a < R; ++a)
+            for (int j = 0; j < cols; ++j)
+              for (int b = 0; b < C; ++b)
+                s[((size_t)(i * R + a)) * (C * cols) + j * C + b] =
+                  A[i * cols + j] * r[(size_t)a * C + b];
+        r.swap(s);
+        R *= rows;
+        C *= cols;
+      }
+    return r;
+  };
+  const std::vector<double> V = tensor(t.S, nq, nd, dim);
+  const std::vector<double> Vf = tensor(t.S, nq, nd, dim - 1);
+  const std::vector<double> P = tensor(t.Sinv, nd, nq, dim);
+  int sd[3] = {1, nq, nq * nq};
+  std::vector<double> X((size_t)np * np), XV((size_t)np * n);
+  std::vector<double> L((size_t)np * nb);
+  for (long long c = 0; c < out.cells; ++c)
+    {
+      const double *ca = &cell[(size_t)c * np * (dim + 1)];
+      const double *fa = &face[(size_t)c * sides * npf];
+      std::fill(X.begin(), X.end(), 0.0);
+      std::fill(L.begin(), L.end(), 0.0);
+      for (int d = 0; d < dim; ++d)
+        {
+          // cell term along the lines of direction d
+          for (int q = 0; q < np; ++q)
+            {
+              const int iq = q / sd[d] % nq, base = q - iq * sd[d];
+              for (int p = 0; p < nq; ++p)
+                {
+                  const int r = base + p * sd[d];
+                  const double cq = ca[(size_t)q * (dim + 1) + d] *
+                                    ca[(size_t)q * (dim + 1) + dim];
+                  const double cr = ca[(size_t)r * (dim + 1) + d] *
+                                    ca[(size_t)r * (dim + 1) + dim];
+                  X[(size_t)q * np + r] +=
+                    (1.0 - skew) * t.Dq[p * nq + iq] * cr -
+                    skew * t.Dq[iq * nq + p] * cq;
+                }
+            }
+          // faces: the own trace where the flow goes out, the neighbour's
+          // values where it comes in
+          for (int side = 0; side < 2; ++side)
+            for (int p = 0; p < npf; ++p)
+              {
+                const double an = fa[(size_t)(2 * d + side) * npf + p];
+                const double own = (an > 0.0 ? an : 0.0) - skew * an;
+                const double in = an < 0.0 ? an : 0.0;
+                const int base = p % sd[d] + (p / sd[d]) * sd[d] * nq;
+                for (int i = 0; i < nq; ++i)
+                  {
+                    const double Fi = t.F[side * nq + i];
+                    const size_t row = (size_t)(base + i * sd[d]);
+                    for (int j = 0; j < nq; ++j)
+                      X[row * np + base + j * sd[d]] -=
+                        Fi * own * t.F[side * nq + j];
+                    for (int b = 0; b < nf; ++b)
+                      L[row * nb + (2 * d + side) * nf + b] -=
+                        Fi * in * Vf[(size_t)p * nf + b];
+                  }
+              }
+        }
+      // inverse mass matrix: divide by JxW, then the projection
+      for (int q = 0; q < np; ++q)
+        {
+          const double s = 1.0 / ca[(size_t)q * (dim + 1) + dim];
+          double *row = &XV[(size_t)q * n];
+          std::fill(row, row + n, 0.0);
+          for (int r = 0; r < np; ++r)
+            {
+              // the lines through q only
+              const double x = X[(size_t)q * np + r] * s;
+              if (x != 0.0)
+                for (int j = 0; j < n; ++j)
+                  row[j] += x * V[(size_t)r * n + j];
+            }
+          for (int b = 0; b < nb; ++b)
+            L[(size_t)q * nb + b] *= s;
+        }
+      double *K = &out.K[(size_t)c * n * n], *B = &out.B[(size_t)c * n * nb];
+      for (int i = 0; i < n; ++i)
+        for (int q = 0; q < np; ++q)
+          {
+            const double w = P[(size_t)i * np + q];
+            for (int j = 0; j < n; ++j)
+              K[(size_t)i * n + j] += w * XV[(size_t)q * n + j];
+            for (int b = 0; b < nb; ++b)
+              B[(size_t)i * nb + b] += w * L[(size_t)q * nb + b];
+          }
     }
 }
 

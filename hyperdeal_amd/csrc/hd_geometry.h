@@ -52,6 +52,26 @@ void space_tables(const SpaceMap &m, int nq, const double *xq,
                   const double *wq, const double *a, std::vector<double> &cell,
                   std::vector<double> &face);
 
+// One space's factor of the constant-velocity operator on a periodic
+// deformed mesh, as dense matrices per cell:
+//   du(i) = sum_j K[cell][i][j] u(j) + sum_q B[cell][i][q] f(q)
+// over the cell's n = nd^dim nodes and the face nodes f of its 2 dim
+// neighbours, q = side nd^(dim-1) + node (side 2 d: the left neighbour across
+// d, its last layer; 2 d + 1: the right one, its first layer).  Built from
+// the operator's tables with the steps of the quadrature algorithm, so that
+// the same quadrature, skew form and inverse mass matrix enter; inflow only
+// (the upwind flux takes the neighbour where a . n < 0).
+struct CurvedHost
+{
+  long long cells = 0;
+  std::vector<double> K; // cells x n x n
+  std::vector<double> B; // cells x n x (2 dim nd^(dim-1))
+};
+struct Tables1D;
+void curved_space_operator(const SpaceMap &m, const Tables1D &t, double skew,
+                           const std::vector<double> &cell,
+                           const std::vector<double> &face, CurvedHost &out);
+
 // largest |(J^{-T} a)_j| over the cells and the points xq of the space
 // (the quantity of the reference's compute_critical_time_step,
 // operators/advection/cfl.h:56-90)

@@ -129,6 +129,9 @@ struct hd_advection
   // cell points, (a . n) JxW_face at the face points) and their view
   double *geo_tab = nullptr;
   hd::DeformDev geo{};
+  // the factorised form of a periodic deformed operator (has_curved: built)
+  hd::CurvedDev curved{};
+  bool has_curved = false;
   bool counted = false; // counted in mf->n_ops
   // Vlasov-Poisson state (velocity (v, grad phi) from the Poisson solve)
   bool vp = false;
