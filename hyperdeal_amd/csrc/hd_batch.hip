@@ -230,8 +230,8 @@ bool valid_ptrs(const hd_batch *b, const void *const *p)
   return true;
 }
 
-// one LSRK step: the FP64 -> precision copy of every solution, then per
-// degree the stages of that degree's operators
+// one LSRK step: the FP64 -> FP32 copy of every solution (FP64: none), then
+// per degree the stages of that degree's operators
 int batch_step(hd_batch *b, const char *type, int precision,
                double *const *sol, void *const *ti_a, void *const *ti_b,
                double dt, const DevPlan &plan, hipStream_t stream)
@@ -242,33 +242,48 @@ int batch_step(hd_batch *b, const char *type, int precision,
     return n_stages;
   const int n = (int)b->ops.size();
   const int pi = prec_index(precision);
+  // FP64: the stages that leave the solution, as in a single-operator step
+  std::vector<int> keep(n_stages, hd::kSolUpdate);
+  if (precision == HD_FP64)
+    hd_abi::deferred_stages(std::vector<double>(a, a + n_stages - 1),
+                            std::vector<double>(bb, bb + n_stages), keep);
+  const bool from_sol = keep[0] == hd::kSolInput;
   hd::BatchPtrs p{};
   for (int i = 0; i < n; ++i)
     {
       p.sol[i] = sol[i];
       p.dst[i] = ti_a[i];
     }
-  hipError_t e = hd::batch_convert(pi, n, b->n_dofs.data(), p, stream);
+  hipError_t e = hipSuccess;
+  if (!from_sol)
+    e = hd::batch_convert(pi, n, b->n_dofs.data(), p, stream);
   if (e != hipSuccess)
     return hip_fail(e, "batch copy");
   e = for_degrees(b, stream, [&](int N, hipStream_t s) {
     hd::BatchPtrs q = p;
-    bool in_a = true;
+    void *const *in = from_sol ? (void *const *)sol : ti_a;
+    void *const *out = from_sol ? ti_a : ti_b;
+    void *const *spare = from_sol ? ti_b : ti_a;
     hipError_t err = hipSuccess;
     for (int st = 0; st < n_stages && err == hipSuccess; ++st)
       {
         const bool last = st == n_stages - 1;
         for (int i = 0; i < n; ++i)
           {
-            q.src[i] = in_a ? ti_a[i] : ti_b[i];
+            q.src[i] = in[i];
             q.dst[i] = nullptr;
-            q.ti[i] = last ? nullptr : (in_a ? ti_b[i] : ti_a[i]);
+            q.ti[i] = last ? nullptr : out[i];
           }
         q.a_dt = last ? 0.0 : a[st] * dt;
         q.b_dt = bb[st] * dt;
+        q.keep = keep[st];
+        q.recover = st > 0 && keep[st - 1] != hd::kSolUpdate
+                      ? bb[st - 1] / a[st - 1]
+                      : 0.0;
         err = hd::collapsed_batch(b->D, N, pi, last ? 2 : 1, b->dev_ops[pi],
                                   plan.tasks[N], plan.plan[N], q, s);
-        in_a = !in_a;
+        in = out;
+        std::swap(out, spare);
       }
     return err;
   });

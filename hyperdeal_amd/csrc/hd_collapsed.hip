@@ -496,7 +496,11 @@ __device__ inline void inflow_cells(long long cell, const MeshDev &mesh,
 
 // MODE 0: dst = apply(src).  MODE 1: LSRK stage with K = apply(src),
 // sol += b_dt K, ti_out = sol_old + a_dt K.  MODE 2: the stage without
-// ti_out (last stage).
+// ti_out (last stage).  FP64 only: MODE 3 and 4, a stage that writes ti_out
+// and leaves sol (StageSol: kSolInput and kSolKeep); MODE 5 and 6, a stage
+// with and without ti_out after such a one (own modes: the input's values
+// stay in registers until the store, which cost the 5 x 5 tiles of the plain
+// stages 4 % as a condition inside them).
 // Resident blocks per CU: LDS allows two (FP64) or four (FP32) 3+3 cells
 // with their R buffers; the FP32 stage keeps the FP64 solution values in
 // registers and runs three to stay clear of spills.  A block of G cells
@@ -707,8 +711,10 @@ apply_block(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ src_,
         const long long g0 = my_cell(c0) * CELL + gbase[p];
         // the stage's solution values go out before the arithmetic (small
         // tiles; large ones load them at the store)
-        constexpr bool kEarlySol = MODE != 0 && NN <= 16;
-        double sv[MODE == 0 ? 1 : NN];
+        constexpr bool kReadsSol = MODE != 0 && MODE != 3;
+        constexpr bool kWritesSol = kReadsSol && MODE != 4;
+        constexpr bool kEarlySol = kReadsSol && NN <= 16;
+        double sv[kReadsSol ? NN : 1];
         if constexpr (kEarlySol)
           {
 #pragma unroll
@@ -731,7 +737,10 @@ apply_block(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ src_,
         face_load<D, N, T, p>(src, gbase[p], nnb, fnode, fc[p]);
         if (store)
           {
-            if constexpr (MODE != 0 && !kEarlySol)
+            // (large tiles read the input's values again from U)
+            if constexpr (kLateLast && (MODE == 3 || MODE == 5 || MODE == 6))
+              tile_read<D, N, T, p>(U, lbase[p], ul);
+            if constexpr (kReadsSol && !kEarlySol)
               {
 #pragma unroll
                 for (int r = 0; r < NN; ++r)
@@ -747,12 +756,21 @@ apply_block(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ src_,
                   __builtin_nontemporal_store(out[r], &dst[g]);
                 else
                   {
-                    __builtin_nontemporal_store(
-                      sv[r] + stage.b_dt * (double)out[r], &sol[g]);
-                    if constexpr (MODE == 1)
+                    // FP64: the input's own values are at hand for a
+                    // solution that the previous stage left
+                    double s;
+                    if constexpr (MODE == 3)
+                      s = (double)ul[r];
+                    else if constexpr (MODE == 5 || MODE == 6)
+                      s = sv[r] + stage.recover * ((double)ul[r] - sv[r]);
+                    else
+                      s = sv[r];
+                    if constexpr (kWritesSol)
                       __builtin_nontemporal_store(
-                        (T)(sv[r] + stage.a_dt * (double)out[r]),
-                        &ti_out[g]);
+                        s + stage.b_dt * (double)out[r], &sol[g]);
+                    if constexpr (MODE != 2 && MODE != 6)
+                      __builtin_nontemporal_store(
+                        (T)(s + stage.a_dt * (double)out[r]), &ti_out[g]);
                   }
               }
           }
@@ -831,6 +849,29 @@ hipError_t launch_g(int mode, const T *src, T *dst, const T *coef,
                        stream, src, dst, coef, mesh, inflow, stage, n_logical,
                        used);
   };
+  if constexpr (sizeof(T) == 8)
+    {
+      if (mode != 0 && stage.keep == kSolInput)
+        {
+          go(apply_kernel<D, N, T, 3, G>, Residency<D, N, T, 3, G>::kBlocks);
+          return hipGetLastError();
+        }
+      if (mode != 0 && stage.keep == kSolKeep)
+        {
+          go(apply_kernel<D, N, T, 4, G>, Residency<D, N, T, 4, G>::kBlocks);
+          return hipGetLastError();
+        }
+      if (mode != 0 && stage.recover != 0.0)
+        {
+          if (stage.ti_out)
+            go(apply_kernel<D, N, T, 5, G>,
+               Residency<D, N, T, 5, G>::kBlocks);
+          else
+            go(apply_kernel<D, N, T, 6, G>,
+               Residency<D, N, T, 6, G>::kBlocks);
+          return hipGetLastError();
+        }
+    }
   const int m = mode == 0 ? 0 : (stage.ti_out ? 1 : 2);
   if (m == 0)
     go(apply_kernel<D, N, T, 0, G>, Residency<D, N, T, 0, G>::kBlocks);
@@ -939,8 +980,10 @@ __global__ __launch_bounds__((Shape<4, N, T, 1>::BLOCK),
       StageDev stage{};
       stage.a_dt = ptrs.a_dt;
       stage.b_dt = ptrs.b_dt;
+      stage.recover = ptrs.recover;
       stage.sol = MODE == 0 ? nullptr : ptrs.sol[op];
-      stage.ti_out = MODE == 1 ? ptrs.ti[op] : nullptr;
+      stage.ti_out =
+        MODE == 0 || MODE == 2 || MODE == 6 ? nullptr : ptrs.ti[op];
       apply_block<4, N, T, MODE, 1>(
         U, R, static_cast<const T *>(ptrs.src[op]),
         MODE == 0 ? static_cast<T *>(ptrs.dst[op]) : nullptr,
@@ -964,6 +1007,27 @@ hipError_t batch_launch(int mode, const BatchOp *ops, const BatchTask *tasks,
                        dim3(Shape<4, N, T, 1>::BLOCK), 0, stream, ops, tasks,
                        plan, ptrs);
   };
+  if constexpr (sizeof(T) == 8)
+    {
+      if (mode == 1 && ptrs.keep == kSolInput)
+        {
+          go(batch_kernel<N, T, 3>);
+          return hipGetLastError();
+        }
+      if (mode == 1 && ptrs.keep == kSolKeep)
+        {
+          go(batch_kernel<N, T, 4>);
+          return hipGetLastError();
+        }
+      if (mode != 0 && ptrs.recover != 0.0)
+        {
+          if (mode == 1)
+            go(batch_kernel<N, T, 5>);
+          else
+            go(batch_kernel<N, T, 6>);
+          return hipGetLastError();
+        }
+    }
   if (mode == 0)
     go(batch_kernel<N, T, 0>);
   else if (mode == 1)
@@ -1229,9 +1293,16 @@ __global__ __launch_bounds__(256, 3) void plane_kernel(
             dst[g] = kq;
           else
             {
-              const double so = stage.sol[g];
-              stage.sol[g] = so + stage.b_dt * (double)kq;
-              if constexpr (MODE == 1)
+              double so;
+              if constexpr (MODE == 3)
+                so = (double)u[q];
+              else if constexpr (MODE == 4 || sizeof(T) == 4)
+                so = stage.sol[g];
+              else
+                so = stage_solution(stage, stage.sol[g], (double)u[q]);
+              if constexpr (MODE == 1 || MODE == 2)
+                stage.sol[g] = so + stage.b_dt * (double)kq;
+              if constexpr (MODE != 2)
                 static_cast<T *>(stage.ti_out)[g] =
                   (T)(so + stage.a_dt * (double)kq);
             }
@@ -1271,6 +1342,21 @@ hipError_t split_launch(int mode, const T *src, T *dst, T *part,
   const long long n = mesh.n_cells * ipow(N, 4);
   const unsigned blocks =
     (unsigned)std::min<long long>((n + 255) / 256, 256LL * 16);
+  if constexpr (sizeof(T) == 8)
+    {
+      if (mode != 0 && stage.keep != kSolUpdate)
+        {
+          if (stage.keep == kSolInput)
+            hipLaunchKernelGGL((plane_kernel<D, N, T, 3>), dim3(blocks),
+                               dim3(256), 0, stream, src, part, dst, coef,
+                               mesh, inflow, stage);
+          else
+            hipLaunchKernelGGL((plane_kernel<D, N, T, 4>), dim3(blocks),
+                               dim3(256), 0, stream, src, part, dst, coef,
+                               mesh, inflow, stage);
+          return hipGetLastError();
+        }
+    }
   if (mode == 0)
     hipLaunchKernelGGL((plane_kernel<D, N, T, 0>), dim3(blocks), dim3(256), 0,
                        stream, src, part, dst, coef, mesh, inflow, stage);

@@ -398,15 +398,27 @@ __global__ __launch_bounds__(kBlock) void curved_kernel(
                     }
                   else
                     {
+                      // (FP64: the input's own values where the solution
+                      // is the input, or is recovered from it)
+                      const bool input =
+                        sizeof(T) == 8 && stage.keep == kSolInput;
 #pragma unroll
                       for (int e = 0; e < 4; ++e)
                         if (in[e])
-                          so[e] = stage.sol[at[e]];
+                          so[e] = input ? (double)src[at[e]]
+                                        : stage.sol[at[e]];
+                      if (sizeof(T) == 8 && stage.recover != 0.0)
 #pragma unroll
-                      for (int e = 0; e < 4; ++e)
-                        if (in[e])
-                          stage.sol[at[e]] =
-                            so[e] + stage.b_dt * (double)acc[r][c][e];
+                        for (int e = 0; e < 4; ++e)
+                          if (in[e])
+                            so[e] = stage_solution(stage, so[e],
+                                                   (double)src[at[e]]);
+                      if (sizeof(T) == 4 || stage.keep == kSolUpdate)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                          if (in[e])
+                            stage.sol[at[e]] =
+                              so[e] + stage.b_dt * (double)acc[r][c][e];
                       if (stage.ti_out)
 #pragma unroll
                         for (int e = 0; e < 4; ++e)

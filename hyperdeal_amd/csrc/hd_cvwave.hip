@@ -248,7 +248,11 @@ cv_block(T *lds, const T *__restrict__ src, T *__restrict__ dst,
       // the solution (LSRK stage), used at the end
       double ps[KU];
       if constexpr (MODE == 1)
-        for_values(n_in, [&](int k, int e) { ps[k] = stage.sol[base + e]; });
+        {
+          // (FP64: a stage whose input is the solution has it in B1)
+          if (sizeof(T) == 4 || stage.keep != kSolInput)
+            for_values(n_in, [&](int k, int e) { ps[k] = stage.sol[base + e]; });
+        }
       // V: K = P + sum over v0, v1, along the lines of this lane's v-plane
       if (busy)
         {
@@ -304,8 +308,15 @@ cv_block(T *lds, const T *__restrict__ src, T *__restrict__ dst,
           dst[base + e] = a;
         else
           {
-            const double so = ps[k];
-            stage.sol[base + e] = so + stage.b_dt * (double)a;
+            double so = ps[k];
+            if constexpr (sizeof(T) == 8)
+              {
+                const double own = lds[lofs(k) + N2 * P];
+                so = stage.keep == kSolInput ? own
+                                             : stage_solution(stage, so, own);
+              }
+            if (sizeof(T) == 4 || stage.keep == kSolUpdate)
+              stage.sol[base + e] = so + stage.b_dt * (double)a;
             if (stage.ti_out)
               static_cast<T *>(stage.ti_out)[base + e] =
                 (T)(so + stage.a_dt * (double)a);
@@ -437,6 +448,8 @@ __global__ __launch_bounds__(64) void batch_kernel(
       StageDev stage{};
       stage.a_dt = ptrs.a_dt;
       stage.b_dt = ptrs.b_dt;
+      stage.recover = ptrs.recover;
+      stage.keep = ptrs.keep;
       stage.sol = MODE == 0 ? nullptr : ptrs.sol[tk.op];
       stage.ti_out = MODE == 1 ? ptrs.ti[tk.op] : nullptr;
       cv_block<N, T, MODE == 0 ? 0 : 1>(

@@ -37,7 +37,20 @@ struct InflowDev
   int side[kMaxDim];
 };
 
-// LSRK stage epilogue: sol += b_dt K; ti_out = sol_old + a_dt K
+// How an FP64 stage of an LSRK step treats the solution.  With Ti' = s + a K
+// and s' = s + b K the solution after a stage is s + (b / a) (Ti' - s): a
+// stage may leave s in memory and write Ti' alone, and the next stage, which
+// holds its own input Ti', forms s' from the two.  Where |b / a| <= 1 the
+// rounding of Ti' enters s' with no more than its own weight.
+enum StageSol
+{
+  kSolUpdate = 0, // sol is read and written
+  kSolKeep = 1,   // sol is read, not written (the next stage recovers it)
+  kSolInput = 2   // as kSolKeep, and the stage's input is the solution
+};
+
+// LSRK stage epilogue: s = sol, or sol + recover (input - sol) after a stage
+// that left sol; sol = s + b_dt K; ti_out = s + a_dt K
 struct StageDev
 {
   double a_dt, b_dt;
@@ -47,7 +60,17 @@ struct StageDev
   // Vlasov-Poisson stages: the kernel writes the density partials of
   // ti_out here (one per v cell and x node), or null
   double *rho_part;
+  double recover; // FP64: b / a of a previous stage that left sol, else 0
+  int keep;       // StageSol (FP64; FP32 stages update sol)
 };
+
+// the FP64 solution a stage continues from: so = sol, own = the stage's input
+// at the same node (recover 0: so itself)
+__device__ inline double stage_solution(const StageDev &st, double so,
+                                        double own)
+{
+  return st.recover == 0.0 ? so : so + st.recover * (own - so);
+}
 
 // blocks are dispatched round-robin over the 8 XCDs; give each XCD a
 // contiguous range of logical blocks so that face neighbours share an L2
@@ -219,6 +242,8 @@ struct BatchPtrs
   double *sol[kBatchMax];
   void *ti[kBatchMax];
   double a_dt, b_dt;
+  double recover; // see StageDev
+  int keep;
 };
 
 // prefix sums of the operators' DoF counts (batched elementwise kernels)

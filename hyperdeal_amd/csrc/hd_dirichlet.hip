@@ -160,8 +160,10 @@ __global__ __launch_bounds__(kBlock) void correct_kernel(
             dst[idx] = (T)((double)dst[idx] + corr);
           else
             {
-              stage.sol[idx] += stage.b_dt * corr;
-              if (MODE == 1)
+              // (MODE 3: a stage that leaves sol)
+              if (MODE != 3)
+                stage.sol[idx] += stage.b_dt * corr;
+              if (MODE == 1 || MODE == 3)
                 {
                   T *ti = static_cast<T *>(stage.ti_out);
                   ti[idx] = (T)((double)ti[idx] + stage.a_dt * corr);
@@ -192,7 +194,10 @@ hipError_t correct(int D, int N, int NQ, int mode, const T *src, T *dst,
       fd.d = d;
       fd.side = inflow.side[d];
       fd.n_layer = mesh.n_cells / mesh.n[d];
-      const int m = mode == 1 && stage.ti_out ? 1 : (mode == 0 ? 0 : 2);
+      const int m = mode == 0                     ? 0
+                    : stage.keep != kSolUpdate ? 3
+                    : stage.ti_out             ? 1
+                                               : 2;
 #define HD_DIR_LAUNCH(MM)                                                      \
   {                                                                            \
     hipError_t e = hipFuncSetAttribute(                                        \
@@ -208,6 +213,8 @@ hipError_t correct(int D, int N, int NQ, int mode, const T *src, T *dst,
         HD_DIR_LAUNCH(0)
       else if (m == 1)
         HD_DIR_LAUNCH(1)
+      else if (m == 3)
+        HD_DIR_LAUNCH(3)
       else
         HD_DIR_LAUNCH(2)
 #undef HD_DIR_LAUNCH

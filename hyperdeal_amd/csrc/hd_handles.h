@@ -8,7 +8,10 @@
 #include "hd_geometry.h"
 #include "hd_tables.h"
 
+#include <algorithm>
+#include <cmath>
 #include <string>
+#include <vector>
 
 namespace hd_abi
 {
@@ -29,6 +32,37 @@ inline int hip_fail(hipError_t e, const char *where)
 inline int ok()
 {
   return HD_OK;
+}
+
+// Which stages of an FP64 LSRK step (a: n - 1 coefficients, b: n) leave the
+// solution in memory (hd::StageSol): the first, whose input is the solution
+// (no copy of it, 16 bytes per value, and no update, 16 more), and of the
+// others the most that are not adjacent, have |b / a| <= 1 and a successor
+// (8 bytes each).  rk45: stages 0 and 3, 128 instead of 168 bytes per value.
+inline void deferred_stages(const std::vector<double> &a,
+                            const std::vector<double> &b,
+                            std::vector<int> &keep)
+{
+  const size_t n = b.size();
+  keep.assign(n, hd::kSolUpdate);
+  if (n < 2)
+    return;
+  // best[s]: stages that can be left from stage s on, stage s free to choose
+  std::vector<int> best(n + 2, 0);
+  auto can = [&](size_t s) {
+    return s + 1 < n && std::fabs(b[s]) <= std::fabs(a[s]);
+  };
+  for (size_t s = n; s-- > 0;)
+    best[s] = can(s) ? std::max(best[s + 1], 1 + best[s + 2]) : best[s + 1];
+  if (!can(0))
+    return;
+  keep[0] = hd::kSolInput;
+  for (size_t s = 2; s < n; ++s)
+    if (can(s) && 1 + best[s + 2] >= best[s + 1] && 1 + best[s + 2] > 0)
+      {
+        keep[s] = hd::kSolKeep;
+        ++s; // the next stage recovers the solution
+      }
 }
 
 inline hipStream_t as_stream(void *s)
