@@ -1375,12 +1375,6 @@ hipError_t split_dispatch(int D, int N, int mode, const T *src, T *dst,
                           const InflowDev &inflow, const StageDev &stage,
                           hipStream_t stream)
 {
-  if (D == 6 && N == 5)
-    return split_launch<6, 5, T>(mode, src, dst, part, coef, mesh, inflow,
-                                 stage, stream);
-  if (D == 6 && N == 6)
-    return split_launch<6, 6, T>(mode, src, dst, part, coef, mesh, inflow,
-                                 stage, stream);
   if (D == 5 && N == 5)
     return split_launch<5, 5, T>(mode, src, dst, part, coef, mesh, inflow,
                                  stage, stream);

@@ -1,25 +1,38 @@
-// hd_cres.hip -- the FP32 collapsed apply and LSRK stage of 3+3 cells that
-// do not fit LDS (k = 4, 5: 5^6 and 6^6 values), in one pass (gfx950).
+// hd_cres.hip -- the collapsed apply and LSRK stage of 3+3 cells that do not
+// fit LDS (k = 4, 5: 5^6 and 6^6 values), in one pass (gfx950).
 //
-// The collapsed operator (section "Collapsed apply" of hd_collapsed.hip) is
-// a sum of 1D operators, one per direction.  One block per cell: thread t
-// owns the 4D points p = t and t + TH of the first four directions and
-// keeps the outputs of all (i4, i5) at its points in registers (2 N^2
-// accumulators: the cell's result lives in the block's registers, 187 KB at
-// k=5 in FP32).  The input streams through LDS one chunk of fixed i5 at a
-// time (N^5 values, double-buffered); per chunk j a thread adds
-//   - along i5: A5[i5][j] u(p, i4, j) to every output plane i5,
-//   - along i4: A4 u(p, ., j) to plane j,
-//   - along d < 4: the 1D operator of direction d on the LDS lines through p
-//     (per-lane rows of the coefficient table, kept in LDS), to plane j,
-// and the inflow face terms b_d f_d (the neighbour's face values from HBM /
-// L2).  Every value of the cell is read from HBM once and written once: 8
-// bytes per DoF for the FP32 apply plus the faces, against about 24 for the
-// two-pass split form.  FP64 does not fit (373 KB of accumulators per
-// cell), so FP64 keeps the split form.
+// The collapsed operator (see hd_collapsed.hip) is a sum of 1D operators, one
+// per direction.  A block works on one cell at a time (k = 5 in FP64: two
+// blocks share a cell, every other output plane each); the cell's result
+// lives in the block's registers and the input streams through LDS one chunk
+// of fixed i5 (N^5 values) at a time:
+//   - thread t owns the chunk's values e = t + m BLOCK and the results
+//     (e, i5) of the block's planes: loading its values it adds
+//     A5[i5][j] u(e) to all of them and writes the values into U (LDS);
+//   - directions 0 to 4, one per phase: a thread reads its lines from U and
+//     adds the line's sums to R (LDS);
+//   - the owners add R to plane j of their results.
+// The inflow faces of d < 5 go from L2 / HBM into registers of the threads
+// that use them, one phase ahead; that of direction 5 enters as one more
+// input plane.
+//
+// What bounds it: the fabric.  Every value is read once and written once,
+// plus one cell's worth of faces (24 bytes per value for the FP64 apply, 12
+// for FP32; the second block's reads of a cell hit the XCD's L2); beside it
+// 16 LDS accesses and 42 multiply-adds per value.  Measured, 6^6 cells: k = 5
+// FP64 apply 20.9 -> 12.1 ms (the two-pass split form moved 48 bytes per
+// value), FP32 11.1 -> 6.6 ms (lines read by every point they pass, 30 LDS
+// accesses), k = 4 FP64 8.6 -> 4.3, FP32 4.5 -> 2.2 ms.  N x N tiles of two
+// directions per phase instead of lines (14 LDS accesses, three phases) need
+// 40 more registers: FP32 7.4 ms, FP64 spills (13.5 to 60 ms).
+//
+// Blocks of an XCD take consecutive cells in step, so that the faces across
+// x0 and x1, whose values are spread over every line of the neighbour, hit
+// its L2.
 #include "hd_device.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace hd
 {
@@ -27,305 +40,345 @@ namespace cres
 {
 template <class T>
 using cptr = const __attribute__((address_space(4))) T *;
+template <class T>
+using gptr = __attribute__((address_space(1))) T *;
 
-template <int N>
-struct Geo
+// orders LDS accesses without draining the loads in flight
+__device__ inline void lds_barrier()
 {
-  static constexpr int NN = N * N;
-  static constexpr int P = NN * NN;              // 4D points per cell
-  static constexpr int TH = (P + 1) / 2;         // threads owning points
-  static constexpr int BLOCK = (TH + 63) / 64 * 64;
-  static constexpr int CH = P * N;               // values per chunk (i5)
-  static constexpr int FC = P;                   // face values per d < 4
-  static constexpr int BUF = CH + 4 * FC;        // LDS floats per chunk
-  static constexpr long long CELL = (long long)CH * N;
-  static constexpr int LPT = (CH + BLOCK - 1) / BLOCK;     // chunk loads
-};
-
-// 4 bytes per lane from the lane's own global address into LDS at
-// dst_wave + lane (dst_wave uniform over the wave): the data goes straight
-// to LDS without registers and lands by the next barrier
-__device__ inline void load_lds(const float *g, float *dst_wave)
-{
-  __builtin_amdgcn_global_load_lds(
-    (const __attribute__((address_space(1))) void *)g,
-    (__attribute__((address_space(3))) void *)dst_wave, 4, 0, 0);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int N, int MODE>
-__global__ __launch_bounds__(Geo<N>::BLOCK) void cres_kernel(
-  const float *__restrict__ src, float *__restrict__ dst,
-  const float *__restrict__ coef, MeshDev mesh, InflowDev inflow,
-  StageDev stage)
+// HALVES blocks share a cell, BLOCK threads, WAVES per SIMD (the register
+// budget 512 / WAVES).  Measured, 6^6 cells, apply: k = 5 FP64 two blocks of
+// 1024 threads 12.1, 768 12.5, 512 13.4 ms, one block (192 registers of
+// results) spills, 26 ms; FP32 one block of 1024 threads 6.6, 768 7.1, 512
+// 7.5, two blocks of 512 6.9 ms; k = 4 FP64 256 threads 4.3, 512 4.7, FP32
+// 256 threads 2.24, 512 2.43 ms (two or three blocks per CU overlap their
+// phases)
+template <int N, class T>
+struct Geo;
+template <>
+struct Geo<6, double>
 {
-  using G = Geo<N>;
-  constexpr int NN = G::NN, P = G::P, TH = G::TH, CH = G::CH;
-  constexpr int LPT = G::LPT, BLOCK = G::BLOCK;
-  constexpr int FC = G::FC, BUF = G::BUF, PN = P / N;
-  constexpr long long CELL = G::CELL;
-  // per chunk: the N^5 values, then the inflow faces of directions 0..3
-  // (face d: the neighbour's values at its face node, indexed by the point
-  // without digit d and by i4)
-  __shared__ __align__(16) float buf[2][BUF];
-  __shared__ float Ad[4][NN + N]; // A_d (rows: output node) and b_d, d < 4
-  const cptr<float> cc = (cptr<float>)coef;
-  for (int e = threadIdx.x; e < 4 * (NN + N); e += BLOCK)
-    (&Ad[0][0])[e] = coef[e];
+  static constexpr int HALVES = 2, BLOCK = 1024, WAVES = 4;
+};
+template <>
+struct Geo<6, float>
+{
+  static constexpr int HALVES = 1, BLOCK = 1024, WAVES = 4;
+};
+template <>
+struct Geo<5, double>
+{
+  static constexpr int HALVES = 1, BLOCK = 256, WAVES = 2;
+};
+template <>
+struct Geo<5, float>
+{
+  static constexpr int HALVES = 1, BLOCK = 256, WAVES = 3;
+};
 
-  constexpr int sd[4] = {1, N, NN, NN * N};
-  // the thread index and what derives from it are recomputed from an
-  // opaque copy per chunk: no lane-dependent addresses held in registers
-  // across the chunk loop
-  int t;
-  bool own[2];
-  int pp[2];
-  auto lane_setup = [&]() {
-    t = (int)threadIdx.x;
-    asm volatile("" : "+v"(t));
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-      {
-        const int p = t + q * TH;
-        own[q] = t < TH && p < P;
-        pp[q] = own[q] ? p : 0;
-      }
-  };
-  lane_setup();
-  // inflow face nodes (the neighbour's last node from the left, first from
-  // the right)
+template <int N, class T, int MODE>
+__global__ __launch_bounds__((Geo<N, T>::BLOCK), (Geo<N, T>::WAVES)) void
+  cres_kernel(const T *__restrict__ src_, T *__restrict__ dst_,
+              const T *__restrict__ coef, MeshDev mesh, InflowDev inflow,
+              StageDev stage)
+{
+  using G = Geo<N, T>;
+  constexpr int BLOCK = G::BLOCK;
+  constexpr int NN = N * N, P = NN * NN, CH = P * N;
+  constexpr long long CELL = (long long)CH * N;
+  constexpr int M = (CH + BLOCK - 1) / BLOCK;   // owned values per chunk
+  constexpr int KL = (P + BLOCK - 1) / BLOCK;   // lines per thread
+  __shared__ __align__(16) T U[CH], R[CH];
+
+  const gptr<const T> src = (gptr<const T>)src_;
+  const gptr<T> dst = (gptr<T>)dst_;
+  const gptr<double> sol = (gptr<double>)stage.sol;
+  const gptr<T> ti_out = (gptr<T>)static_cast<T *>(stage.ti_out);
+  cptr<T> cc = (cptr<T>)coef;
+  constexpr int DC = NN + N; // coefficients per direction: A_d, b_d
   int fnode[6];
 #pragma unroll
   for (int d = 0; d < 6; ++d)
     fnode[d] = inflow.side[d] < 0 ? 0 : N - 1;
-  // coefficients of the last two directions (uniform: scalar loads)
-  auto A4 = [&](int i, int k) -> float { return cc[4 * (NN + N) + i * N + k]; };
-  auto B4 = [&](int i) -> float { return cc[4 * (NN + N) + NN + i]; };
-  auto A5 = [&](int i, int k) -> float { return cc[5 * (NN + N) + i * N + k]; };
-  auto B5 = [&](int i) -> float { return cc[5 * (NN + N) + NN + i]; };
-  __syncthreads();
 
-  // the inflow neighbours of a cell (uniform over the block)
-  struct Nb
-  {
-    long long d0, d1, d2, d3, d4, d5;
+  // consecutive cells per XCD (blocks are dispatched round-robin over them);
+  // HALVES blocks share a cell: block h keeps the planes i5 = h, h + HALVES,
+  // .. and takes the other planes of the input for direction 5 only, from
+  // the L2 that the other block's loads have filled (step is even, so h is
+  // the block's own)
+  constexpr int HALVES = G::HALVES, NPL = (N + HALVES - 1) / HALVES;
+  static_assert(N % HALVES == 0, "planes per block");
+  const long long per = (mesh.n_cells + 7) / 8 * HALVES;
+  const long long u_end =
+    min(mesh.n_cells * HALVES, (long long)(blockIdx.x % 8 + 1) * per);
+  const int step = gridDim.x / 8;
+  long long unit = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (unit >= u_end)
+    return; // uniform for the block, before any barrier
+  const int h = (int)(unit % HALVES);
+
+  // the lane index, made opaque per phase: addresses derived from it are
+  // recomputed instead of held in registers across the chunk loop
+  auto lane = [&]() {
+    unsigned t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
   };
-  auto neighbours = [&](long long cl) -> Nb {
-    Nb r;
-    r.d0 = inflow_neighbour(mesh, cl, 0, inflow.side[0]);
-    r.d1 = inflow_neighbour(mesh, cl, 1, inflow.side[1]);
-    r.d2 = inflow_neighbour(mesh, cl, 2, inflow.side[2]);
-    r.d3 = inflow_neighbour(mesh, cl, 3, inflow.side[3]);
-    r.d4 = inflow_neighbour(mesh, cl, 4, inflow.side[4]);
-    r.d5 = inflow_neighbour(mesh, cl, 5, inflow.side[5]);
-    return r;
-  };
-  // chunk j of a cell and its faces into LDS buffer b, straight from HBM /
-  // L2 (element e of a wave lands at the wave's base + lane).  Face d of
-  // the chunk: the neighbour's values at its face node, indexed by the point
-  // without digit d and by i4; one direction per pass, so that no
-  // lane-dependent choice of neighbour is needed
-  constexpr int FPD = (FC + BLOCK - 1) / BLOCK;
-  auto fetch = [&](long long cl, const Nb &nbx, int j, int b) {
-    const int wbase = t & ~63;
-    const float *uc = src + cl * CELL;
+  auto values = [&](gptr<const T> from, T *v) {
+    const unsigned t = lane();
 #pragma unroll
-    for (int l = 0; l < LPT; ++l)
+    for (int m = 0; m < M; ++m)
       {
-        const int e = t + BLOCK * l;
-        if (e < CH)
-          load_lds(uc + (long long)CH * j + e, &buf[b][wbase + BLOCK * l]);
-      }
-#pragma unroll
-    for (int d = 0; d < 4; ++d)
-      {
-        const long long nbd = d == 0   ? nbx.d0
-                              : d == 1 ? nbx.d1
-                              : d == 2 ? nbx.d2
-                                       : nbx.d3;
-        const float *fsrc =
-          src + nbd * CELL + (long long)fnode[d] * sd[d] + (long long)CH * j;
-#pragma unroll
-        for (int l = 0; l < FPD; ++l)
-          {
-            const int e = t + BLOCK * l;
-            if (e < FC)
-              {
-                const int c = e % PN, i4 = e / PN;
-                const int pf = c % sd[d] + sd[d] * N * (c / sd[d]);
-                load_lds(fsrc + pf + (long long)P * i4,
-                         &buf[b][CH + d * FC + wbase + BLOCK * l]);
-              }
-          }
+        // (uniform base, 32-bit lane offset)
+        const gptr<const T> base = from + m * BLOCK;
+        const unsigned e =
+          m + 1 < M ? t : min(t, (unsigned)(CH - 1 - m * BLOCK));
+        v[m] = base[e];
       }
   };
 
-  // the first cell's first chunk; every later cell's first chunk goes out
-  // before the previous cell's outputs
-  Nb nb{};
-  if ((long long)blockIdx.x < mesh.n_cells)
+  typedef T Planes __attribute__((ext_vector_type(NPL)));
+  Planes acc[M];
+  T pu[M]; // the next chunk's own values
+  values(src + unit / HALVES * CELL, pu);
+  for (; unit < u_end; unit += step)
     {
-      nb = neighbours(blockIdx.x);
-      fetch(blockIdx.x, nb, 0, 0);
-    }
-  for (long long cell = blockIdx.x; cell < mesh.n_cells; cell += gridDim.x)
-    {
-      float acc[2][N][N]; // [point][i4][i5]
+      const long long cell = unit / HALVES;
+      long long nb[6];
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
+      for (int d = 0; d < 6; ++d)
+        nb[d] = inflow_neighbour(mesh, cell, d, inflow.side[d]);
+      {
+        // the inflow face across direction 5: one more input plane
+        const cptr<T> b5 = cc + 5 * DC + NN;
+        const unsigned t = lane();
+        const gptr<const T> s5 = src + nb[5] * CELL + (long long)CH * fnode[5];
 #pragma unroll
-        for (int a = 0; a < N; ++a)
-#pragma unroll
-          for (int b = 0; b < N; ++b)
-            acc[q][a][b] = 0.0f;
-      // the i4 and i5 inflow faces of this thread's points go out now and
-      // land with the first chunk (no global load inside the chunk loop)
-      float f4[2][N], f5[2][N];
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int k = 0; k < N; ++k)
+        for (int m0 = 0; m0 < M; m0 += 4)
           {
-            f4[q][k] = src[nb.d4 * CELL + pp[q] + (long long)P * (fnode[4] + N * k)];
-            f5[q][k] = src[nb.d5 * CELL + pp[q] + (long long)P * (k + N * fnode[5])];
-          }
-      __syncthreads();
+            // four values in flight at a time (registers)
+            T f5[4];
 #pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (m0 + e < M)
+                {
+                  constexpr int last = CH - 1 - (M - 1) * BLOCK;
+                  const gptr<const T> base = s5 + (m0 + e) * BLOCK;
+                  f5[e] =
+                    base[m0 + e + 1 < M ? t : min(t, (unsigned)last)];
+                }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (m0 + e < M)
+#pragma unroll
+                for (int i = 0; i < NPL; ++i)
+                  acc[m0 + e < M ? m0 + e : M - 1][i] =
+                    b5[h + HALVES * i] * f5[e];
+          }
+      }
       for (int j = 0; j < N; ++j)
         {
-          // the next chunk travels into the other buffer meanwhile (every
-          // thread finished reading it before the barrier that ended the
-          // previous chunk)
-          lane_setup();
-          if (j + 1 < N)
-            fetch(cell, nb, j + 1, (j + 1) & 1);
-          const float *ch = buf[j & 1];
+          asm volatile("" : "+s"(cc));
+          // the inflow values of this thread's lines along d, and the lines:
+          // sums into R (d = 0) or added
+          auto line_faces = [&](auto dc, T *f) {
+            constexpr int d = decltype(dc)::value, sd = ipow(N, d);
+            const unsigned t = lane();
+            const gptr<const T> s =
+              src + nb[d] * CELL + (long long)CH * j + fnode[d] * sd;
 #pragma unroll
-          for (int q = 0; q < 2; ++q)
+            for (int k = 0; k < KL; ++k)
+              {
+                const unsigned l = min(t + k * BLOCK, (unsigned)(P - 1));
+                f[k] = s[l % sd + l / sd * (unsigned)(sd * N)];
+              }
+          };
+          auto lines = [&](auto dc, const T *f) {
+            constexpr int d = decltype(dc)::value, sd = ipow(N, d);
+            const unsigned t = lane();
+            const cptr<T> A = cc + d * DC, bv = A + NN;
+#pragma unroll
+            for (int k = 0; k < KL; ++k)
+              {
+                const unsigned l = t + k * BLOCK;
+                if (P % BLOCK != 0 && k + 1 == KL && l >= P)
+                  continue;
+                const unsigned base = l % sd + l / sd * (unsigned)(sd * N);
+                T u[N];
+#pragma unroll
+                for (int i = 0; i < N; ++i)
+                  u[i] = U[base + i * sd];
+#pragma unroll
+                for (int i = 0; i < N; ++i)
+                  {
+                    T s = bv[i] * f[k];
+#pragma unroll
+                    for (int q = 0; q < N; ++q)
+                      s += A[i * N + q] * u[q];
+                    T *r = &R[base + i * sd];
+                    *r = d == 0 ? s : *r + s;
+                  }
+              }
+          };
+          using D0 = std::integral_constant<int, 0>;
+          using D1 = std::integral_constant<int, 1>;
+          using D2 = std::integral_constant<int, 2>;
+          using D3 = std::integral_constant<int, 3>;
+          using D4 = std::integral_constant<int, 4>;
+
+          // 1) own values: direction 5, and into U
+          const bool mine = HALVES == 1 || j % HALVES == h;
+          T f0[KL], f1[KL];
+          if (mine)
+            line_faces(D0(), f0);
+          {
+            const unsigned t = lane();
+            const cptr<T> A5 = cc + 5 * DC + j + h * N;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+              {
+#pragma unroll
+                for (int i = 0; i < NPL; ++i)
+                  acc[m][i] += A5[i * HALVES * N] * pu[m];
+                if (mine &&
+                    (CH % BLOCK == 0 || m + 1 < M || t + m * BLOCK < CH))
+                  U[t + m * BLOCK] = pu[m];
+              }
+          }
+          // the next chunk: of this cell, or the next cell's first
+          const long long nc =
+            j + 1 < N ? cell
+                      : (unit + step < u_end ? (unit + step) / HALVES : cell);
+          const gptr<const T> next =
+            src + nc * CELL + (long long)CH * (j + 1 < N ? j + 1 : 0);
+          if (!mine)
             {
-              if (!own[q])
-                continue;
-              const int p = pp[q];
-              float v[N];
-#pragma unroll
-              for (int k = 0; k < N; ++k)
-                v[k] = ch[p + P * k];
-              // along i5: plane j of the input feeds every output plane
-#pragma unroll
-              for (int i5 = 0; i5 < N; ++i5)
-                {
-                  const float a5 = A5(i5, j);
-#pragma unroll
-                  for (int i4 = 0; i4 < N; ++i4)
-                    acc[q][i4][i5] += a5 * v[i4];
-                }
-              // along i4, within plane j, with the i4 inflow face
-#pragma unroll
-              for (int i4 = 0; i4 < N; ++i4)
-                {
-                  float a = B4(i4) * f4[q][j];
-#pragma unroll
-                  for (int k = 0; k < N; ++k)
-                    a += A4(i4, k) * v[k];
-                  acc[q][i4][j] += a;
-                }
-              // along d < 4: the lines through p in the LDS chunk
-#pragma unroll
-              for (int d = 0; d < 4; ++d)
-                {
-                  const int row = (p / sd[d]) % N;
-                  const int base = p - row * sd[d];
-                  const float *ar = &Ad[d][row * N];
-                  const float br = Ad[d][NN + row];
-                  // face index of p in direction d: p without its digit d
-                  const int pc = p % sd[d] + sd[d] * (p / (sd[d] * N));
-                  const float *fd = ch + CH + d * FC + pc;
-#pragma unroll
-                  for (int i4 = 0; i4 < N; ++i4)
-                    {
-                      float a = br * fd[PN * i4];
-#pragma unroll
-                      for (int k = 0; k < N; ++k)
-                        a += ar[k] * ch[base + k * sd[d] + P * i4];
-                      acc[q][i4][j] += a;
-                    }
-                }
+              values(next, pu);
+              continue;
             }
-          // the next chunk's loads have landed and this chunk's reads are
-          // done (the barrier waits for both)
-          __syncthreads();
-        }
-      // the next cell's first chunk travels while this cell's outputs go
-      // out (both buffers are free after the last chunk's barrier); then
-      // the outputs with the i5 inflow face (for fixed (i4, i5) the points
-      // of consecutive threads are consecutive values)
-      const long long next = cell + gridDim.x;
-      if (next < mesh.n_cells)
-        {
-          lane_setup();
-          nb = neighbours(next);
-          fetch(next, nb, 0, 0);
-        }
+          lds_barrier();
+          values(next, pu);
+          // 2) the lines of directions 0 to 3, the faces one ahead
+          line_faces(D1(), f1);
+          lines(D0(), f0);
+          lds_barrier();
+          line_faces(D2(), f0);
+          lines(D1(), f1);
+          lds_barrier();
+          line_faces(D3(), f1);
+          lines(D2(), f0);
+          lds_barrier();
+          line_faces(D4(), f0);
+          lines(D3(), f1);
+          lds_barrier();
+          lines(D4(), f0);
+          lds_barrier();
+          // 3) the chunk's sums into plane j (the next chunk's U may be
+          // written meanwhile: nobody reads U before the next barrier)
+          {
+            const unsigned t = lane();
+            // (j is uniform: plane j of a register vector is one indexed
+            // access; a switch over j kept two copies of every result)
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
+            for (int m = 0; m < M; ++m)
+              if (CH % BLOCK == 0 || m + 1 < M || t + m * BLOCK < CH)
+                acc[m][j / HALVES] += R[t + m * BLOCK];
+          }
+        }
+      // the results (e, i5): coalesced, not read again by this kernel
+      const unsigned t = lane();
+#pragma unroll
+      for (int m = 0; m < M; ++m)
         {
-          if (!own[q])
+          if (!(CH % BLOCK == 0 || m + 1 < M || t + m * BLOCK < CH))
             continue;
-          const int p = pp[q];
-          const long long g0 = cell * CELL + p;
+          constexpr bool kReadsSol = MODE != 0 && MODE != 3;
+          constexpr bool kOwn = MODE == 3 || MODE == 5 || MODE == 6;
+          double so[kReadsSol ? NPL : 1], own[kOwn ? NPL : 1];
 #pragma unroll
-          for (int i4 = 0; i4 < N; ++i4)
+          for (int i = 0; i < NPL; ++i)
             {
-              // a stage's solution values of this i4 row: N loads in flight
-              // before the first store
-              double so[MODE == 0 ? 1 : N];
-              if constexpr (MODE != 0)
+              const long long g = cell * CELL + m * BLOCK +
+                                  (long long)CH * (h + HALVES * i);
+              if constexpr (kReadsSol)
+                so[i] = (sol + g)[t];
+              if constexpr (kOwn)
+                own[i] = (double)(src + g)[t];
+            }
 #pragma unroll
-                for (int i5 = 0; i5 < N; ++i5)
-                  so[i5] = stage.sol[g0 + (long long)P * (i4 + N * i5)];
-#pragma unroll
-              for (int i5 = 0; i5 < N; ++i5)
+          for (int i = 0; i < NPL; ++i)
+            {
+              const long long g = cell * CELL + m * BLOCK +
+                                  (long long)CH * (h + HALVES * i);
+              const T k = acc[m][i];
+              if constexpr (MODE == 0)
+                __builtin_nontemporal_store(k, &(dst + g)[t]);
+              else
                 {
-                  const float k = acc[q][i4][i5] + B5(i5) * f5[q][i4];
-                  const long long g = g0 + (long long)P * (i4 + N * i5);
-                  if constexpr (MODE == 0)
-                    dst[g] = k;
+                  double s;
+                  if constexpr (MODE == 3)
+                    s = own[i];
+                  else if constexpr (MODE == 5 || MODE == 6)
+                    s = so[i] + stage.recover * (own[i] - so[i]);
                   else
-                    {
-                      stage.sol[g] = so[i5] + stage.b_dt * (double)k;
-                      if constexpr (MODE == 1)
-                        static_cast<float *>(stage.ti_out)[g] =
-                          (float)(so[i5] + stage.a_dt * (double)k);
-                    }
+                    s = so[i];
+                  if constexpr (kReadsSol && MODE != 4)
+                    __builtin_nontemporal_store(s + stage.b_dt * (double)k,
+                                                &(sol + g)[t]);
+                  if constexpr (MODE != 2 && MODE != 6)
+                    __builtin_nontemporal_store(
+                      (T)(s + stage.a_dt * (double)k), &(ti_out + g)[t]);
                 }
             }
         }
     }
 }
 
-template <int N>
-hipError_t launch(int mode, const float *src, float *dst, const float *coef,
+template <int N, class T>
+hipError_t launch(int mode, const T *src, T *dst, const T *coef,
                   const MeshDev &mesh, const InflowDev &inflow,
                   const StageDev &stage, hipStream_t stream)
 {
+  using G = Geo<N, T>;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
                             dev) != hipSuccess ||
-      cus < 1)
+      cus < 8)
     cus = 256;
-  const unsigned grid =
-    (unsigned)std::min<long long>(mesh.n_cells, (long long)cus);
-  const dim3 block(Geo<N>::BLOCK);
+  auto go = [&](auto kernel) {
+    // as many persistent blocks as are resident, a multiple of the XCDs
+    int bpc = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, kernel, G::BLOCK,
+                                                     0) != hipSuccess ||
+        bpc < 1)
+      bpc = 1;
+    const long long most = (mesh.n_cells + 7) / 8 * 8 * G::HALVES;
+    const unsigned grid = (unsigned)std::min<long long>(
+      most, (long long)(cus * bpc) / (8 * G::HALVES) * (8 * G::HALVES));
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(G::BLOCK), 0, stream, src,
+                       dst, coef, mesh, inflow, stage);
+    return hipGetLastError();
+  };
   if (mode == 0)
-    hipLaunchKernelGGL((cres_kernel<N, 0>), dim3(grid), block, 0, stream,
-                       src, dst, coef, mesh, inflow, stage);
-  else if (stage.ti_out)
-    hipLaunchKernelGGL((cres_kernel<N, 1>), dim3(grid), block, 0, stream,
-                       src, dst, coef, mesh, inflow, stage);
-  else
-    hipLaunchKernelGGL((cres_kernel<N, 2>), dim3(grid), block, 0, stream,
-                       src, dst, coef, mesh, inflow, stage);
-  return hipGetLastError();
+    return go(cres_kernel<N, T, 0>);
+  if constexpr (sizeof(T) == 8)
+    {
+      if (stage.keep == kSolInput)
+        return go(cres_kernel<N, T, 3>);
+      if (stage.keep == kSolKeep)
+        return go(cres_kernel<N, T, 4>);
+      if (stage.recover != 0.0)
+        return stage.ti_out ? go(cres_kernel<N, T, 5>)
+                            : go(cres_kernel<N, T, 6>);
+    }
+  return stage.ti_out ? go(cres_kernel<N, T, 1>) : go(cres_kernel<N, T, 2>);
 }
 } // namespace cres
 
@@ -334,15 +387,25 @@ bool collapsed_cres_supported(int D, int N)
   return D == 6 && (N == 5 || N == 6);
 }
 
+hipError_t collapsed_cres_f64(int N, int mode, const double *src, double *dst,
+                              const double *coef, const MeshDev &mesh,
+                              const InflowDev &inflow, const StageDev &stage,
+                              hipStream_t stream)
+{
+  return N == 5 ? cres::launch<5>(mode, src, dst, coef, mesh, inflow, stage,
+                                  stream)
+                : cres::launch<6>(mode, src, dst, coef, mesh, inflow, stage,
+                                  stream);
+}
+
 hipError_t collapsed_cres_f32(int N, int mode, const float *src, float *dst,
                               const float *coef, const MeshDev &mesh,
                               const InflowDev &inflow, const StageDev &stage,
                               hipStream_t stream)
 {
-  if (N == 5)
-    return cres::launch<5>(mode, src, dst, coef, mesh, inflow, stage, stream);
-  if (N == 6)
-    return cres::launch<6>(mode, src, dst, coef, mesh, inflow, stage, stream);
-  return hipErrorInvalidValue;
+  return N == 5 ? cres::launch<5>(mode, src, dst, coef, mesh, inflow, stage,
+                                  stream)
+                : cres::launch<6>(mode, src, dst, coef, mesh, inflow, stage,
+                                  stream);
 }
 } // namespace hd

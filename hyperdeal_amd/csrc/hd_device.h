@@ -308,9 +308,13 @@ hipError_t collapsed_split_f32(int D, int N, int mode, const float *src,
                                float *dst, float *part, const float *coef,
                                const MeshDev &mesh, const InflowDev &inflow,
                                const StageDev &stage, hipStream_t stream);
-// FP32 3+3 cells larger than LDS in one pass, the cell's result held in a
+// 3+3 cells larger than LDS in one pass, the cell's result held in a
 // block's registers (hd_cres.hip)
 bool collapsed_cres_supported(int D, int N);
+hipError_t collapsed_cres_f64(int N, int mode, const double *src, double *dst,
+                              const double *coef, const MeshDev &mesh,
+                              const InflowDev &inflow, const StageDev &stage,
+                              hipStream_t stream);
 hipError_t collapsed_cres_f32(int N, int mode, const float *src, float *dst,
                               const float *coef, const MeshDev &mesh,
                               const InflowDev &inflow, const StageDev &stage,
