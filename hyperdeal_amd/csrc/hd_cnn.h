@@ -54,7 +54,9 @@ struct CnnNet
   hipError_t pack(hipStream_t s);
   hipError_t reserve(int batch);
   // out = net(in); in, out: batch x H x W
-  hipError_t forward(const float *in, float *out, int batch, hipStream_t s);
+  // keep: the activations stay for a backward pass
+  hipError_t forward(const float *in, float *out, int batch, hipStream_t s,
+                     bool keep = false);
   // loss = mean (net(in) - target)^2 into loss_dev, gradient into grad
   hipError_t loss_and_grad(const float *in, const float *target, int batch,
                            hipStream_t s);

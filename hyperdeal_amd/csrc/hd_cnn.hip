@@ -56,11 +56,13 @@ __device__ inline int wrap(int i, int n)
 // out[b][o] = act(bias[o] + sum_{i,k} w[i][k][o] in[b][i] shifted by k),
 // w packed as [CIN][9][COUT rounded up to even] BF16.  Grid
 // (W / 16, H / 16, batch * COUT / OT), one output pixel and OT channels per
-// thread.
+// thread.  act (input gradients, not ACT): the layer input's activations (they
+// have the signs of the pre-activations), by whose leaky ReLU the gradient goes on.
 template <int CIN, int COUT, bool ACT>
 __global__ __launch_bounds__(kTile *kTile) void conv_kernel(
   const float *__restrict__ in, const uint32_t *__restrict__ w,
-  const float *__restrict__ bias, float *__restrict__ out, int H, int W)
+  const float *__restrict__ bias, float *__restrict__ out, int H, int W,
+  const float *__restrict__ act)
 {
   constexpr int OT = COUT < 8 ? COUT : 8;
   constexpr int NG = COUT / OT;
@@ -116,7 +118,11 @@ __global__ __launch_bounds__(kTile *kTile) void conv_kernel(
       float v = acc[o] + (bias ? ((cptr<float>)bias)[oc] : 0.0f);
       if (ACT)
         v = v > 0.0f ? v : kSlope * v;
-      out[((long long)b * COUT + oc) * plane + (long long)y * W + x] = v;
+      const long long at =
+        ((long long)b * COUT + oc) * plane + (long long)y * W + x;
+      if (!ACT && act)
+        v *= act[at] > 0.0f ? 1.0f : kSlope;
+      out[at] = v;
     }
 }
 
@@ -151,10 +157,16 @@ constexpr int kWStride = 304;    // >= 9 * 32 = 288
 // without further barriers (dynamic LDS: kConvLds bytes).
 constexpr int kConvLds =
   kChannels * (kTileStride + kWStride) * (int)sizeof(float);
-template <bool ACT, int OH>
+// FIRST (inference): `in` is the one-channel image, and the block forms its
+// input tile itself, the 1 -> 32 layer with weights w0 and biases b0 (same
+// order of sums as conv_kernel): one launch and one pass over 32 channels
+// less.
+template <bool ACT, int OH, bool FIRST>
 __global__ __launch_bounds__(256) void conv32_mfma_kernel(
   const float *__restrict__ in, const uint32_t *__restrict__ w,
-  const float *__restrict__ bias, float *__restrict__ out, int H, int W)
+  const float *__restrict__ bias, float *__restrict__ out, int H, int W,
+  const float *__restrict__ act, const uint32_t *__restrict__ w0,
+  const float *__restrict__ b0)
 {
   constexpr int C = kChannels;
   constexpr int WPR = C / 2;        // packed words per (input channel, tap)
@@ -169,6 +181,47 @@ __global__ __launch_bounds__(256) void conv32_mfma_kernel(
   const int b = blockIdx.z / OH, half = blockIdx.z % OH;
   const int x0 = blockIdx.x * kMTX, y0 = blockIdx.y * kMTY;
   const long long plane = (long long)H * W;
+  if constexpr (FIRST)
+    {
+      constexpr int IX = kMTX + 4, IY = kMTY + 4;
+      __shared__ float img[IY * IX];
+      for (int e = threadIdx.x; e < IY * IX; e += 256)
+        img[e] = in[(long long)b * plane +
+                    (long long)wrap(y0 + e / IX - 2, H) * W +
+                    wrap(x0 + e % IX - 2, W)];
+      __syncthreads();
+      // a wave's lanes are pixels, its channels uniform
+      const cptr<uint32_t> wc = (cptr<uint32_t>)w0;
+      for (int r = lane; r < HW; r += 64)
+        {
+          float v[9];
+#pragma unroll
+          for (int k = 0; k < 9; ++k)
+            v[k] = img[(r / (kMTX + 2) + k / 3) * IX + r % (kMTX + 2) + k % 3];
+#pragma unroll
+          for (int j = 0; j < C / 8; ++j)
+            {
+              const int pr = __builtin_amdgcn_readfirstlane(wave) * (C / 8) + j;
+              float lo = 0.0f, hi = 0.0f;
+#pragma unroll
+              for (int k = 0; k < 9; ++k)
+                {
+                  const uint32_t u = wc[k * (C / 2) + pr];
+                  lo += bits_to_float(u << 16) * v[k];
+                  hi += bits_to_float(u & 0xffff0000u) * v[k];
+                }
+              lo += ((cptr<float>)b0)[2 * pr];
+              hi += ((cptr<float>)b0)[2 * pr + 1];
+              tile[2 * pr * kTileStride + r] = lo > 0.0f ? lo : kSlope * lo;
+              tile[(2 * pr + 1) * kTileStride + r] =
+                hi > 0.0f ? hi : kSlope * hi;
+            }
+        }
+    }
+  else
+  // (the copies are unrolled: their loads are in flight together, one round
+  // trip instead of one per value)
+#pragma unroll 12
   for (int e = threadIdx.x; e < C * HW; e += 256)
     {
       const int i = e / HW, r = e % HW;
@@ -177,6 +230,7 @@ __global__ __launch_bounds__(256) void conv32_mfma_kernel(
       tile[i * kTileStride + r] =
         in[((long long)b * C + i) * plane + (long long)yy * W + xx];
     }
+#pragma unroll 9
   for (int e = threadIdx.x; e < C * 9 * WPH; e += 256)
     {
       const int i = e / (9 * WPH), r = e % (9 * WPH);
@@ -196,7 +250,7 @@ __global__ __launch_bounds__(256) void conv32_mfma_kernel(
   for (int tap = 0; tap < 9; ++tap)
     {
       const int dy = tap / 3, dx = tap % 3;
-#pragma unroll 2
+#pragma unroll OH == 2 ? 8 : 2
       for (int q = 0; q < C / 4; ++q)
         {
           const int ci = q * 4 + k4;
@@ -230,7 +284,11 @@ __global__ __launch_bounds__(256) void conv32_mfma_kernel(
           if (ACT)
             v = v > 0.0f ? v : kSlope * v;
           const int y = y0 + wave * 2 + r, x = x0 + n16;
-          out[((long long)b * C + oc) * plane + (long long)y * W + x] = v;
+          const long long at =
+            ((long long)b * C + oc) * plane + (long long)y * W + x;
+          if (!ACT && act)
+            v *= act[at] > 0.0f ? 1.0f : kSlope;
+          out[at] = v;
         }
 }
 
@@ -287,14 +345,17 @@ __global__ __launch_bounds__(256) void conv_to1_kernel(
 // Weight gradient of a 32 -> 32 layer: gw[o][i][tap] = sum over the batch
 // and pixels of g[o][pixel] in[i][pixel + tap]; a GEMM with M = 32 (o),
 // N = 288 (i, tap), K = pixels.  Block p sums the 16 x 16 pixel tiles p,
-// p + gridDim.x, ... into part[p][o][i][tap] (wave w owns the N tiles
-// w, w + 4, ... of the 18, for both M tiles); the blocks' partials are then
-// added in a fixed order (part_reduce_kernel), so the result is
-// deterministic.
+// p + gridDim.x, ... into part[p][o][i][tap]: waves w and w + 4 own the N
+// tiles w, w + 4, ... of the 18 (for both M tiles), each over one half of the
+// pixels, and the halves are added through LDS (a block has a compute unit
+// to itself: two waves per SIMD hide each other's LDS latency); the
+// blocks' partials are then added in a fixed order (part_reduce_kernel), so
+// the result is deterministic.
 constexpr int kGStride = 272;   // 256 pixels of one gradient channel, +16
 constexpr int kWgradOut = kChannels * kChannels * 9 + kChannels; // per block
 constexpr int kInStride = 336;  // 18 x 18 = 324 input pixels, 336 = 16 mod 64
-__global__ __launch_bounds__(256) void wgrad32_mfma_kernel(
+constexpr int kWgradThreads = 512;
+__global__ __launch_bounds__(kWgradThreads) void wgrad32_mfma_kernel(
   const float *__restrict__ in, const float *__restrict__ g,
   float *__restrict__ part, int B, int H, int W)
 {
@@ -303,7 +364,8 @@ __global__ __launch_bounds__(256) void wgrad32_mfma_kernel(
   extern __shared__ float sm[];
   float *gs = sm;                  // [C][kGStride]
   float *is = sm + C * kGStride;   // [C][kInStride]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = (threadIdx.x >> 6) & 3, half = threadIdx.x >> 8;
   const int n16 = lane & 15, k4 = lane >> 4;
   const int tx = W / 16, ty = H / 16;
   const long long n_tiles = (long long)B * tx * ty;
@@ -323,13 +385,15 @@ __global__ __launch_bounds__(256) void wgrad32_mfma_kernel(
       const int rem = (int)(t % (tx * ty));
       const int y0 = (rem / tx) * 16, x0 = (rem % tx) * 16;
       __syncthreads(); // the previous tile's LDS reads are done
-      for (int e = threadIdx.x; e < C * 256; e += 256)
+#pragma unroll 16
+      for (int e = threadIdx.x; e < C * 256; e += kWgradThreads)
         {
           const int o = e / 256, p = e % 256;
           gs[o * kGStride + p] = g[((long long)b * C + o) * plane +
                                    (long long)(y0 + p / 16) * W + x0 + p % 16];
         }
-      for (int e = threadIdx.x; e < C * 324; e += 256)
+#pragma unroll 7
+      for (int e = threadIdx.x; e < C * 324; e += kWgradThreads)
         {
           const int i = e / 324, r = e % 324;
           const int yy = wrap(y0 + r / 18 - 1, H), xx = wrap(x0 + r % 18 - 1, W);
@@ -337,16 +401,18 @@ __global__ __launch_bounds__(256) void wgrad32_mfma_kernel(
             in[((long long)b * C + i) * plane + (long long)yy * W + xx];
         }
       __syncthreads();
-      // this thread's share of the bias gradient: channel t / 8, pixels
-      // 32 (t % 8) .. + 31 of the tile
+      // this thread's share of the bias gradient: channel t / 16, pixels
+      // t % 16, + 16, ... of the tile
       {
-        const float *gr = gs + (threadIdx.x / 8) * kGStride + 32 * (threadIdx.x % 8);
-#pragma unroll 8
-        for (int j = 0; j < 32; ++j)
-          bsum += gr[j];
+        const float *gr =
+          gs + (threadIdx.x / 16) * kGStride + threadIdx.x % 16;
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          bsum += gr[16 * j];
       }
       // K steps of 4 pixels: pixel p = 4 s + k4 of the tile
-      for (int s = 0; s < 64; ++s)
+#pragma unroll 4
+      for (int s = 32 * half; s < 32 * half + 32; ++s)
         {
           const int p = 4 * s + k4;
           const int py = p / 16, px = p % 16;
@@ -374,15 +440,31 @@ __global__ __launch_bounds__(256) void wgrad32_mfma_kernel(
   // bias gradient's block partials after them: part[block][C * C * 9 + o]
   float *pb = part + (long long)blockIdx.x * kWgradOut;
   {
-    __shared__ float bred[256];
+    __shared__ float bred[kWgradThreads];
     bred[threadIdx.x] = bsum;
+    __syncthreads(); // and the last tile's LDS reads are done
+    // the upper half's sums over the staged tiles
+    float *hs = sm + ((wave * 2 * NW) * 64 + lane) * 4;
+    if (half == 1)
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          *reinterpret_cast<mfma_f4 *>(hs + (m * NW + j) * 256) = acc[m][j];
     __syncthreads();
+    if (half == 1)
+      return;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int j = 0; j < NW; ++j)
+        acc[m][j] += *reinterpret_cast<const mfma_f4 *>(hs + (m * NW + j) * 256);
     if (threadIdx.x < C)
       {
         float t = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          t += bred[threadIdx.x * 8 + j];
+        for (int j = 0; j < 16; ++j)
+          t += bred[threadIdx.x * 16 + j];
         pb[C * C * 9 + threadIdx.x] = t;
       }
   }
@@ -411,6 +493,7 @@ __global__ __launch_bounds__(256) void part_reduce_kernel(
   const int o = blockIdx.x * 64 + threadIdx.x % 64, q = threadIdx.x / 64;
   float s = 0.0f;
   if (o < n_out)
+#pragma unroll 16
     for (int p = q; p < n_part; p += 4)
       s += part[(long long)p * n_out + o];
   red[q][threadIdx.x % 64] = s;
@@ -548,16 +631,6 @@ __global__ void mse_finish_kernel(const double *__restrict__ partial, int nb,
     }
 }
 
-// g *= leaky-ReLU'(pre-activation); a is the post-activation output, which
-// has the sign of the pre-activation
-__global__ void act_grad_kernel(float *__restrict__ g,
-                                const float *__restrict__ a, long long n)
-{
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    g[i] *= a[i] > 0.0f ? 1.0f : kSlope;
-}
-
 // Adam on the FP32 master parameters (bias-corrected step sizes c1, c2)
 __global__ void adam_kernel(float *__restrict__ p, float *__restrict__ m,
                             float *__restrict__ v,
@@ -576,11 +649,20 @@ __global__ void adam_kernel(float *__restrict__ p, float *__restrict__ m,
     }
 }
 
-// master weights w[Co][Ci][9] of one layer -> the two packed BF16 copies
-__global__ void pack_kernel(const float *__restrict__ w, int Ci, int Co,
-                            uint32_t *__restrict__ fwd,
-                            uint32_t *__restrict__ bwd)
+// master weights w[Co][Ci][9] of a layer (grid row) -> the two packed BF16
+// copies
+struct PackLayers
 {
+  const float *w[kLayers];
+  uint32_t *fwd[kLayers], *bwd[kLayers];
+  int Ci[kLayers], Co[kLayers];
+};
+__global__ void pack_kernel(PackLayers layers)
+{
+  const float *__restrict__ w = layers.w[blockIdx.y];
+  uint32_t *__restrict__ fwd = layers.fwd[blockIdx.y];
+  uint32_t *__restrict__ bwd = layers.bwd[blockIdx.y];
+  const int Ci = layers.Ci[blockIdx.y], Co = layers.Co[blockIdx.y];
   const int wpo = (Co + 1) / 2, wpi = (Ci + 1) / 2;
   const int n_f = Ci * 9 * wpo, n_b = Co * 9 * wpi;
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n_f + n_b;
@@ -873,14 +955,20 @@ void CnnNet::release()
 
 hipError_t CnnNet::pack(hipStream_t s)
 {
+  cnn::PackLayers a{};
+  int most = 0;
   for (int l = 0; l < cnn::kLayers; ++l)
     {
-      const int n = fwd_words(l) + bwd_words(l);
-      hipLaunchKernelGGL(cnn::pack_kernel, dim3((n + 255) / 256), dim3(256), 0,
-                         s, p + param_offset_w(l), in_channels(l),
-                         out_channels(l), pk + pack_offset_fwd(l),
-                         pk + pack_offset_bwd(l));
+      a.w[l] = p + param_offset_w(l);
+      a.fwd[l] = pk + pack_offset_fwd(l);
+      a.bwd[l] = pk + pack_offset_bwd(l);
+      a.Ci[l] = in_channels(l);
+      a.Co[l] = out_channels(l);
+      most = std::max(most, fwd_words(l) + bwd_words(l));
     }
+  hipLaunchKernelGGL(cnn::pack_kernel,
+                     dim3((most + 255) / 256, cnn::kLayers), dim3(256), 0, s,
+                     a);
   return hipGetLastError();
 }
 
@@ -935,29 +1023,32 @@ Bufs buffers(float *act, int nb, int H, int W)
 
 template <int CIN, int COUT, bool ACT>
 void conv(const float *in, const uint32_t *w, const float *bias, float *out,
-          int batch, int H, int W, hipStream_t s)
+          int batch, int H, int W, hipStream_t s, const float *act = nullptr)
 {
   constexpr int OT = COUT < 8 ? COUT : 8;
   hipLaunchKernelGGL((cnn::conv_kernel<CIN, COUT, ACT>),
                      dim3(W / cnn::kTile, H / cnn::kTile,
                           batch * (COUT / OT)),
                      dim3(cnn::kTile * cnn::kTile), 0, s, in, w, bias, out, H,
-                     W);
+                     W, act);
 }
 
-template <bool ACT, int OH>
+template <bool ACT, int OH, bool FIRST = false>
 hipError_t conv32_launch(const float *in, const uint32_t *w,
                          const float *bias, float *out, int batch, int H,
-                         int W, hipStream_t s)
+                         int W, hipStream_t s, const float *act,
+                         const uint32_t *w0 = nullptr,
+                         const float *b0 = nullptr)
 {
   hipError_t e = hipFuncSetAttribute(
-    reinterpret_cast<const void *>(&cnn::conv32_mfma_kernel<ACT, OH>),
+    reinterpret_cast<const void *>(&cnn::conv32_mfma_kernel<ACT, OH, FIRST>),
     hipFuncAttributeMaxDynamicSharedMemorySize, cnn::kConvLds);
   if (e != hipSuccess)
     return e;
-  hipLaunchKernelGGL((cnn::conv32_mfma_kernel<ACT, OH>),
+  hipLaunchKernelGGL((cnn::conv32_mfma_kernel<ACT, OH, FIRST>),
                      dim3(W / cnn::kMTX, H / cnn::kMTY, batch * OH),
-                     dim3(256), cnn::kConvLds, s, in, w, bias, out, H, W);
+                     dim3(256), cnn::kConvLds, s, in, w, bias, out, H, W,
+                     act, w0, b0);
   return hipGetLastError();
 }
 
@@ -965,12 +1056,13 @@ hipError_t conv32_launch(const float *in, const uint32_t *w,
 // so that a 128 x 128 image still fills the GPU's CUs
 template <bool ACT>
 hipError_t conv32(const float *in, const uint32_t *w, const float *bias,
-                  float *out, int batch, int H, int W, hipStream_t s)
+                  float *out, int batch, int H, int W, hipStream_t s,
+                  const float *act = nullptr)
 {
   const long long tiles = (long long)batch * (H / cnn::kMTY) * (W / cnn::kMTX);
   return tiles < 512
-           ? conv32_launch<ACT, 2>(in, w, bias, out, batch, H, W, s)
-           : conv32_launch<ACT, 1>(in, w, bias, out, batch, H, W, s);
+           ? conv32_launch<ACT, 2>(in, w, bias, out, batch, H, W, s, act)
+           : conv32_launch<ACT, 1>(in, w, bias, out, batch, H, W, s, act);
 }
 
 void conv_to1(const float *in, const uint32_t *w, const float *bias,
@@ -993,8 +1085,8 @@ hipError_t wgrad32(const float *in, const float *g, float *part, float *gw,
   if (e != hipSuccess)
     return e;
   const int nb = wgrad_blocks(batch, H, W);
-  hipLaunchKernelGGL(cnn::wgrad32_mfma_kernel, dim3(nb), dim3(256), lds, s,
-                     in, g, part, batch, H, W);
+  hipLaunchKernelGGL(cnn::wgrad32_mfma_kernel, dim3(nb),
+                     dim3(cnn::kWgradThreads), lds, s, in, g, part, batch, H, W);
   const int n_out = cnn::kWgradOut;
   // gw and gb are adjacent in the parameter layout (w[Co][Ci][9], b[Co])
   hipLaunchKernelGGL(cnn::part_reduce_kernel, dim3((n_out + 63) / 64),
@@ -1017,26 +1109,28 @@ hipError_t wgrad_split(const float *in, const float *g, float *part,
                      kSplitChunks, CIN, pairs, gw, gb);
   return hipGetLastError();
 }
-
-void act_grad(float *g, const float *a, long long n, hipStream_t s)
-{
-  const unsigned blocks = (unsigned)std::min<long long>((n + 255) / 256, 8192);
-  hipLaunchKernelGGL(cnn::act_grad_kernel, dim3(blocks), dim3(256), 0, s, g, a,
-                     n);
-}
 } // namespace
 
 hipError_t CnnNet::forward(const float *in, float *out, int batch,
-                           hipStream_t s)
+                           hipStream_t s, bool keep)
 {
   hipError_t e = reserve(batch);
   if (e != hipSuccess)
     return e;
   const Bufs b = buffers(act, batch, H, W);
-  conv<1, 32, true>(in, pk + pack_offset_fwd(0), p + param_offset_b(0), b.a1,
-                    batch, H, W, s);
-  e = conv32<true>(b.a1, pk + pack_offset_fwd(1), p + param_offset_b(1), b.a2,
-                   batch, H, W, s);
+  // without a backward pass a small batch forms the first layer inside the
+  // second
+  if (!keep && (long long)batch * (H / cnn::kMTY) * (W / cnn::kMTX) < 512)
+    e = conv32_launch<true, 2, true>(
+      in, pk + pack_offset_fwd(1), p + param_offset_b(1), b.a2, batch, H, W, s,
+      nullptr, pk + pack_offset_fwd(0), p + param_offset_b(0));
+  else
+    {
+      conv<1, 32, true>(in, pk + pack_offset_fwd(0), p + param_offset_b(0),
+                        b.a1, batch, H, W, s);
+      e = conv32<true>(b.a1, pk + pack_offset_fwd(1), p + param_offset_b(1),
+                       b.a2, batch, H, W, s);
+    }
   if (e == hipSuccess)
     e = conv32<true>(b.a2, pk + pack_offset_fwd(2), p + param_offset_b(2),
                      b.a3, batch, H, W, s);
@@ -1054,11 +1148,10 @@ hipError_t CnnNet::loss_and_grad(const float *in, const float *target,
   if (e != hipSuccess)
     return e;
   const Bufs b = buffers(act, batch, H, W);
-  e = forward(in, b.out, batch, s);
+  e = forward(in, b.out, batch, s, true);
   if (e != hipSuccess)
     return e;
   const long long plane = (long long)H * W;
-  const long long nC = (long long)batch * cnn::kChannels * plane;
   const int C = cnn::kChannels;
   // the loss partials sit in the weight-gradient buffer, consumed at once
   double *mse_part = reinterpret_cast<double *>(part);
@@ -1073,28 +1166,25 @@ hipError_t CnnNet::loss_and_grad(const float *in, const float *target,
   if (e != hipSuccess)
     return e;
   conv<1, 32, false>(b.g0, pk + pack_offset_bwd(3), nullptr, b.g1, batch, H, W,
-                     s);
-  act_grad(b.g1, b.a3, nC, s);
+                     s, b.a3);
   // layer 2
   e = wgrad32(b.a2, b.g1, part, grad + param_offset_w(2),
               grad + param_offset_b(2), batch, H, W, s);
   if (e != hipSuccess)
     return e;
   e = conv32<false>(b.g1, pk + pack_offset_bwd(2), nullptr, b.g0, batch, H, W,
-                    s);
+                    s, b.a2);
   if (e != hipSuccess)
     return e;
-  act_grad(b.g0, b.a2, nC, s);
   // layer 1
   e = wgrad32(b.a1, b.g0, part, grad + param_offset_w(1),
               grad + param_offset_b(1), batch, H, W, s);
   if (e != hipSuccess)
     return e;
   e = conv32<false>(b.g0, pk + pack_offset_bwd(1), nullptr, b.g1, batch, H, W,
-                    s);
+                    s, b.a1);
   if (e != hipSuccess)
     return e;
-  act_grad(b.g1, b.a1, nC, s);
   // layer 0 (1 -> C)
   return wgrad_split<1, 32>(in, b.g1, part, grad + param_offset_w(0),
                             grad + param_offset_b(0), batch, H, W, s);
