@@ -86,11 +86,17 @@ int vp_update(hd_advection *op, const double *f, const float *f32,
       e = hd::vp_fdm_solve(*op->fdm, op->ptab, op->rho, stream);
       guess = op->fdm->x;
     }
+  hd::GuessImage image;
+  if (guess && op->learned && op->strips)
+    {
+      image.image = op->learned->img_out;
+      image.scale = op->learned->scale;
+    }
   if (e == hipSuccess)
     e = hd::vp_poisson(op->xdev, op->mf->nd, op->rho, op->phi, guess,
                        op->efield, op->work, op->poisson_tol,
                        op->poisson_max_it, op->stats, stream, op->ptab,
-                       nullptr, !op->learned && op->fdm_on);
+                       nullptr, !op->learned && op->fdm_on, op->strips, image);
   if (e == hipSuccess && op->learned)
     e = hd_abi::learned_after_solve(*op, stream);
   return e == hipSuccess ? HD_OK : hip_fail(e, "Vlasov-Poisson field update");
@@ -698,7 +704,7 @@ int hd_advection_destroy(hd_advection *op)
                   (void *)op->rho, (void *)op->phi, (void *)op->work,
                   (void *)op->partial, (void *)op->stats,
                   (void *)op->ptab, (void *)op->vtab, (void *)op->rho_part,
-                  op->split_scratch, (void *)op->geo_tab})
+                  op->strips, op->split_scratch, (void *)op->geo_tab})
     if (p)
       (void)hipFree(p);
   if (op->mf && op->mf->n_ops > 0 && op->counted)
@@ -933,6 +939,13 @@ int hd_vlasov_poisson_create(hd_matrix_free *mf, double skew_factor,
       if (e == hipSuccess)
         e = hipMemcpy(op->ptab, tab.data(), tab.size() * sizeof(double),
                       hipMemcpyHostToDevice);
+      if (e == hipSuccess &&
+          hd::vp_strips_supported(mf->dim_x, nd, op->xdev.n))
+        {
+          e = hipMalloc(&op->strips, hd::vp_strips_bytes(nd, op->xdev.n));
+          if (e == hipSuccess)
+            e = hd::vp_strips_reset(op->strips, nd, op->xdev.n);
+        }
     }
   if (e != hipSuccess)
     {

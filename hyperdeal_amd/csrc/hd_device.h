@@ -429,13 +429,36 @@ struct ResidualImage
 {
   float *image = nullptr;  // (n1 N) x (n0 N) floats
   double *scale = nullptr; // one double
+  double *phi_copy = nullptr; // several-workgroup form: phi is copied here
+};
+// A guess that is still an image of the x nodes (the learned start's network
+// output; the layout of cnn_image_to_dofs, which is what it stands for)
+struct GuessImage
+{
+  const float *image = nullptr;
+  const double *scale = nullptr;
 };
 hipError_t vp_poisson(const XDev &xd, int N, const double *rho, double *phi,
                       const double *guess, double *efield, double *work,
                       double rel_tol, int max_it, long long *stats,
                       hipStream_t stream, const double *tab2d = nullptr,
                       const ResidualImage *residual = nullptr,
-                      bool guess_alone = false);
+                      bool guess_alone = false, void *strips = nullptr,
+                      const GuessImage &guess_image = GuessImage());
+// the 2D solve on several workgroups (hd_vpcg.hip), in strips of x cell rows:
+// strips: vp_strips_bytes of device memory, reset once, that one solve at a
+// time uses; the mark (0 / 1: a workgroup gave up) sits behind its slots
+bool vp_strips_supported(int dim_x, int N, const int *n);
+size_t vp_strips_bytes(int N, const int *n);
+hipError_t vp_strips_reset(void *comm, int N, const int *n);
+hipError_t vp_strips_solve(const XDev &xd, int N, const double *rho,
+                           double *phi, const double *guess, double *efield,
+                           double *work, void *comm, double rel_tol,
+                           int max_it,
+                           long long *stats, hipStream_t stream,
+                           const double *tab2d, bool guess_alone,
+                           const ResidualImage *residual,
+                           const GuessImage &guess_image);
 bool vp_poisson2d_supported(int dim_x, int N, long long n_x_cells);
 // the 2+2 Vlasov-Poisson apply with the velocity (v, grad phi): a table of
 // vp_apply_table_size(N) doubles, then the same values as floats (the

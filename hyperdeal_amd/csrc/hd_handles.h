@@ -135,7 +135,7 @@ struct hd_learned_guess
   // training runs on its own stream while the solve's CG (one workgroup)
   // runs on the caller's: forked after the guess, joined before the next
   hipStream_t train_stream = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_done = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_phi = nullptr, ev_done = nullptr;
   bool pending = false; // training enqueued and not yet joined
 };
 
@@ -180,6 +180,7 @@ struct hd_advection
          *partial = nullptr;
   long long *stats = nullptr; // solver statistics, see hd::vp_poisson
   double *ptab = nullptr;     // 2D SIPG table of the fast solver, or null
+  void *strips = nullptr;     // inboxes of its several-workgroup form, or null
   double *vtab = nullptr;     // tables of the 2+2 phase-space apply, or null
   double *rho_part = nullptr; // density partials written by a stage
   hd_learned_guess *learned = nullptr;

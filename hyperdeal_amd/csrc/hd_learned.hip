@@ -54,7 +54,7 @@ hipError_t learned_before_solve(hd_advection &op, const double **guess,
       lg.pending = false;
     }
   const size_t bytes = (size_t)op.n_x_dofs * sizeof(double);
-  if (e == hipSuccess)
+  if (e == hipSuccess && !op.strips)
     e = hipMemcpyAsync(lg.phi_prev, op.phi, bytes, hipMemcpyDeviceToDevice,
                        s);
   // the residual image straight from the solver's kernel
@@ -62,14 +62,16 @@ hipError_t learned_before_solve(hd_advection &op, const double **guess,
   hd::ResidualImage resid;
   resid.image = slot;
   resid.scale = lg.scale;
+  resid.phi_copy = op.strips ? lg.phi_prev : nullptr;
   if (e == hipSuccess)
     e = hd::vp_poisson(op.xdev, op.mf->nd, op.rho, op.phi, nullptr,
                        op.efield, op.work, op.poisson_tol, op.poisson_max_it,
-                       op.stats, s, op.ptab, &resid);
+                       op.stats, s, op.ptab, &resid, false, op.strips);
   if (e == hipSuccess && lg.cnn.net.steps > 0)
     {
       e = lg.cnn.net.forward(slot, lg.img_out, 1, s);
-      if (e == hipSuccess)
+      // (the several-workgroup solver takes the image itself)
+      if (e == hipSuccess && !op.strips)
         e = hd::cnn_image_to_dofs(lg.img_out, lg.scale, lg.n0, lg.n1, lg.N,
                                   lg.guess, s);
       if (e == hipSuccess)
@@ -80,44 +82,43 @@ hipError_t learned_before_solve(hd_advection &op, const double **guess,
     }
   if (e != hipSuccess)
     return e;
-  // training on the complete pairs (every slot but the head, which this
-  // solve fills), overlapped with the CG
-  const long long n = lg.solves + 1;
-  const int every = n <= lg.dense_solves ? 1 : lg.train_every;
-  const bool full = lg.count == lg.capacity;
-  const int complete = full ? lg.capacity - 1 : lg.count;
-  if (every <= 0 || complete < lg.min_pairs || complete < 1 || n % every != 0)
-    return hipSuccess;
-  e = hipEventRecord(lg.ev_fork, s);
-  if (e == hipSuccess)
-    e = hipStreamWaitEvent(lg.train_stream, lg.ev_fork, 0);
-  for (int t = 0; t < lg.train_steps && e == hipSuccess; ++t)
-    {
-      e = hd::cnn_sample(lg.ring_in, lg.ring_tgt, lg.seed, lg.draws, complete,
-                         full ? lg.head : -1, lg.train_batch, lg.plane,
-                         lg.batch_in, lg.batch_tgt, lg.train_stream);
-      lg.draws += (uint64_t)lg.train_batch;
-      if (e == hipSuccess)
-        e = lg.cnn.net.loss_and_grad(lg.batch_in, lg.batch_tgt,
-                                     lg.train_batch, lg.train_stream);
-      if (e == hipSuccess)
-        e = lg.cnn.net.adam(lg.lr, lg.train_stream);
-    }
-  if (e == hipSuccess)
-    e = hipEventRecord(lg.ev_done, lg.train_stream);
-  if (e == hipSuccess)
-    lg.pending = true;
-  return e;
+  // the training of this solve starts from here
+  return hipEventRecord(lg.ev_fork, s);
 }
 
 hipError_t learned_after_solve(hd_advection &op, hipStream_t s)
 {
   hd_learned_guess &lg = *op.learned;
+  hipError_t e = hipEventRecord(lg.ev_phi, s);
+  // training on the complete pairs (every slot but the head, which this
+  // solve fills), beside the CG: enqueued after it, so that its three dozen
+  // launches do not hold the CG's back
+  const long long n = lg.solves + 1;
+  const int every = n <= lg.dense_solves ? 1 : lg.train_every;
+  const bool full = lg.count == lg.capacity;
+  const int complete = full ? lg.capacity - 1 : lg.count;
+  if (e == hipSuccess && every > 0 && complete >= lg.min_pairs &&
+      complete >= 1 && n % every == 0)
+    {
+      e = hipStreamWaitEvent(lg.train_stream, lg.ev_fork, 0);
+      for (int t = 0; t < lg.train_steps && e == hipSuccess; ++t)
+        {
+          e = hd::cnn_sample(lg.ring_in, lg.ring_tgt, lg.seed, lg.draws,
+                             complete, full ? lg.head : -1, lg.train_batch,
+                             lg.plane, lg.batch_in, lg.batch_tgt,
+                             lg.train_stream);
+          lg.draws += (uint64_t)lg.train_batch;
+          if (e == hipSuccess)
+            e = lg.cnn.net.loss_and_grad(lg.batch_in, lg.batch_tgt,
+                                         lg.train_batch, lg.train_stream);
+          if (e == hipSuccess)
+            e = lg.cnn.net.adam(lg.lr, lg.train_stream);
+        }
+    }
   // the target image on the training stream too: phi and phi_prev stay as
   // they are until the next solve, which joins that stream first
-  hipError_t e = hipEventRecord(lg.ev_fork, s);
   if (e == hipSuccess)
-    e = hipStreamWaitEvent(lg.train_stream, lg.ev_fork, 0);
+    e = hipStreamWaitEvent(lg.train_stream, lg.ev_phi, 0);
   if (e == hipSuccess)
     e = hd::cnn_dofs_to_image(op.phi, lg.phi_prev, lg.n0, lg.n1, lg.N,
                               lg.ring_tgt + (long long)lg.head * lg.plane,
@@ -148,6 +149,8 @@ void learned_release(hd_learned_guess *lg)
     (void)hipFree(p);
   if (lg->ev_fork)
     (void)hipEventDestroy(lg->ev_fork);
+  if (lg->ev_phi)
+    (void)hipEventDestroy(lg->ev_phi);
   if (lg->ev_done)
     (void)hipEventDestroy(lg->ev_done);
   if (lg->train_stream)
@@ -368,6 +371,8 @@ int hd_vp_learned_guess_enable(hd_advection *op, unsigned long long seed,
     e = hipStreamCreateWithFlags(&lg->train_stream, hipStreamNonBlocking);
   if (e == hipSuccess)
     e = hipEventCreateWithFlags(&lg->ev_fork, hipEventDisableTiming);
+  if (e == hipSuccess)
+    e = hipEventCreateWithFlags(&lg->ev_phi, hipEventDisableTiming);
   if (e == hipSuccess)
     e = hipEventCreateWithFlags(&lg->ev_done, hipEventDisableTiming);
   if (e == hipSuccess)

@@ -1129,13 +1129,18 @@ hipError_t vp_poisson(const XDev &xd, int N, const double *rho, double *phi,
                       const double *guess, double *efield, double *work,
                       double rel_tol, int max_it, long long *stats,
                       hipStream_t stream, const double *tab2d,
-                      const ResidualImage *residual, bool guess_alone)
+                      const ResidualImage *residual, bool guess_alone,
+                      void *strips, const GuessImage &guess_image)
 {
   if (residual &&
       !(tab2d && vp_poisson2d_supported(xd.dim, N, xd.n_cells)))
     return hipErrorInvalidValue;
   if (tab2d && vp_poisson2d_supported(xd.dim, N, xd.n_cells))
     {
+      if (strips)
+        return vp_strips_solve(xd, N, rho, phi, guess, efield, work, strips,
+                               rel_tol, max_it, stats, stream, tab2d,
+                               guess_alone, residual, guess_image);
       const size_t lds =
         (size_t)(vlasov::kPStride * N * N + 32) * sizeof(double);
 #define HD_VP2(NN_)                                                            \
