@@ -67,10 +67,18 @@ bool vp_kernel_active(const hd_advection *op)
 
 // rho (from f, or from the partials of the previous stage), the potential
 // solve (with the learned guess when it is on), grad phi
+// mixed: for an FP32 apply or stage.  Those solve on one workgroup unless the
+// start is the exact one: the learned start, made for them, trains on the
+// rest of the GPU meanwhile, and its step may cost no more than 1.02 of the
+// previous-potential step's.  On strips that does not hold in every run, as
+// CG is then hardly dearer than the network (32^4 cells, k = 3, ms per step
+// with the previous potential and learned: one workgroup 14.4 and 13.9,
+// strips 10.0 and 10.15, of which one run in twelve was over the limit).
 int vp_update(hd_advection *op, const double *f, const float *f32,
-              hipStream_t stream, bool from_partials = false,
+              hipStream_t stream, bool mixed, bool from_partials = false,
               bool rho_ready = false)
 {
+  void *strips = mixed && !op->fdm_on ? nullptr : op->strips;
   hipError_t e =
     rho_ready ? hipSuccess
     : from_partials
@@ -80,14 +88,14 @@ int vp_update(hd_advection *op, const double *f, const float *f32,
                        op->partial, op->density_chunks, op->rho, stream);
   const double *guess = nullptr;
   if (e == hipSuccess && op->learned)
-    e = hd_abi::learned_before_solve(*op, &guess, stream);
+    e = hd_abi::learned_before_solve(*op, &guess, strips, stream);
   else if (e == hipSuccess && op->fdm_on)
     {
       e = hd::vp_fdm_solve(*op->fdm, op->ptab, op->rho, stream);
       guess = op->fdm->x;
     }
   hd::GuessImage image;
-  if (guess && op->learned && op->strips)
+  if (guess && op->learned && strips)
     {
       image.image = op->learned->img_out;
       image.scale = op->learned->scale;
@@ -96,7 +104,7 @@ int vp_update(hd_advection *op, const double *f, const float *f32,
     e = hd::vp_poisson(op->xdev, op->mf->nd, op->rho, op->phi, guess,
                        op->efield, op->work, op->poisson_tol,
                        op->poisson_max_it, op->stats, stream, op->ptab,
-                       nullptr, !op->learned && op->fdm_on, op->strips, image);
+                       nullptr, !op->learned && op->fdm_on, strips, image);
   if (e == hipSuccess && op->learned)
     e = hd_abi::learned_after_solve(*op, stream);
   return e == hipSuccess ? HD_OK : hip_fail(e, "Vlasov-Poisson field update");
@@ -113,16 +121,19 @@ int run_operator(hd_advection *op, int mode, int precision, const void *src,
   if (op->vp && op->vp_auto)
     {
       int rc;
+      const bool mixed = precision != HD_FP64;
       if (density == kDensityReady)
-        rc = vp_update(op, nullptr, nullptr, stream, false, true);
+        rc = vp_update(op, nullptr, nullptr, stream, mixed, false, true);
       else if (density == kDensityPartials)
-        rc = vp_update(op, nullptr, nullptr, stream, true);
+        rc = vp_update(op, nullptr, nullptr, stream, mixed, true);
       else if (density == kDensitySolution)
-        rc = vp_update(op, sol, nullptr, stream);
-      else if (precision == HD_FP64)
-        rc = vp_update(op, static_cast<const double *>(src), nullptr, stream);
+        rc = vp_update(op, sol, nullptr, stream, mixed);
+      else if (!mixed)
+        rc = vp_update(op, static_cast<const double *>(src), nullptr, stream,
+                       mixed);
       else
-        rc = vp_update(op, nullptr, static_cast<const float *>(src), stream);
+        rc = vp_update(op, nullptr, static_cast<const float *>(src), stream,
+                       mixed);
       if (rc != HD_OK)
         return rc;
     }
@@ -961,7 +972,7 @@ int hd_vp_update_field(hd_advection *op, const double *f, void *stream)
   if (!op || !f || !op->vp)
     return fail(HD_ERR_INVALID, "hd_vp_update_field: not a Vlasov-Poisson "
                                 "operator or null argument");
-  return vp_update(op, f, nullptr, as_stream(stream));
+  return vp_update(op, f, nullptr, as_stream(stream), false);
 }
 
 int hd_vp_set_auto_update(hd_advection *op, int enable)

@@ -196,7 +196,7 @@ namespace hd_abi
 // x-space DoFs; returns the guess or null) and after it (training pair,
 // scheduled training steps); rho must be current
 hipError_t learned_before_solve(hd_advection &op, const double **guess,
-                                hipStream_t s);
+                                void *strips, hipStream_t s);
 hipError_t learned_after_solve(hd_advection &op, hipStream_t s);
 void learned_release(hd_learned_guess *lg);
 } // namespace hd_abi

@@ -40,7 +40,7 @@ using hd_abi::as_stream;
 namespace hd_abi
 {
 hipError_t learned_before_solve(hd_advection &op, const double **guess,
-                                hipStream_t s)
+                                void *strips, hipStream_t s)
 {
   hd_learned_guess &lg = *op.learned;
   *guess = nullptr;
@@ -54,7 +54,7 @@ hipError_t learned_before_solve(hd_advection &op, const double **guess,
       lg.pending = false;
     }
   const size_t bytes = (size_t)op.n_x_dofs * sizeof(double);
-  if (e == hipSuccess && !op.strips)
+  if (e == hipSuccess && !strips)
     e = hipMemcpyAsync(lg.phi_prev, op.phi, bytes, hipMemcpyDeviceToDevice,
                        s);
   // the residual image straight from the solver's kernel
@@ -62,16 +62,16 @@ hipError_t learned_before_solve(hd_advection &op, const double **guess,
   hd::ResidualImage resid;
   resid.image = slot;
   resid.scale = lg.scale;
-  resid.phi_copy = op.strips ? lg.phi_prev : nullptr;
+  resid.phi_copy = strips ? lg.phi_prev : nullptr;
   if (e == hipSuccess)
     e = hd::vp_poisson(op.xdev, op.mf->nd, op.rho, op.phi, nullptr,
                        op.efield, op.work, op.poisson_tol, op.poisson_max_it,
-                       op.stats, s, op.ptab, &resid, false, op.strips);
+                       op.stats, s, op.ptab, &resid, false, strips);
   if (e == hipSuccess && lg.cnn.net.steps > 0)
     {
       e = lg.cnn.net.forward(slot, lg.img_out, 1, s);
       // (the several-workgroup solver takes the image itself)
-      if (e == hipSuccess && !op.strips)
+      if (e == hipSuccess && !strips)
         e = hd::cnn_image_to_dofs(lg.img_out, lg.scale, lg.n0, lg.n1, lg.N,
                                   lg.guess, s);
       if (e == hipSuccess)
