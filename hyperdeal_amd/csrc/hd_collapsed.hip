@@ -1212,8 +1212,8 @@ hipError_t batch_convert(int precision, int n_ops, const long long *n_dofs,
 }
 
 // ---------------------------------------------------------------------------
-// Split form for cells larger than LDS (3+3 at k = 5: 6^6 values, 373 KB in
-// FP64).  The collapsed operator is a sum of 1D operators, one per
+// Split form for 5D cells at k = 4 and 5 (6D cells of these degrees take one
+// pass, hd_cres.hip).  The collapsed operator is a sum of 1D operators, one per
 // direction, so it splits exactly:
 //   part = sum_{d < 4} (A_d u along d + b_d face_d)
 //          the 4D kernel, unchanged, on the slabs of fixed (i4, ..): a slab

@@ -21,8 +21,8 @@
 // solves, train_steps Adam steps on batches drawn on the device from the
 // ring's complete pairs.  The training and the target image run on a stream
 // of their own, forked after the guess (and after the CG) and joined before
-// the next solve: the CG of a solve runs in one workgroup, so the rest of
-// the GPU trains meanwhile.
+// the next solve: the CG of a solve runs in one workgroup (32 at most, in
+// FP64 steps), so the rest of the GPU trains meanwhile.
 // The network learns the shape of A^-1 on the residuals this run produces;
 // the combination sets the scale.  Nothing here synchronises with the host.
 #include "hd_handles.h"
