@@ -14,6 +14,13 @@
 // own rows of p, s, x, r and its copy of the neighbours' rows of s and r by
 // the same recurrences.
 //
+// A has the constants as its null space.  CG cannot lower the mean that
+// rounding leaves in r, and once r is no larger than that, steps along the
+// constants (den near 0) make r grow without bound: at 4 x 96 cells, k = 3
+// and a tolerance of 1e-13, below the 2e-11 that b - A x reaches in 64 bits,
+// solves ended at 1e-5.  So r's mean is removed every kProject iterations;
+// b - A x then stays where it is for any tolerance.
+//
 // The exchange.  Every value has a slot of its own in the receiving
 // workgroup's inbox (relaxed agent-scope 8-byte atomics, which the level-2
 // caches of the XCDs do not hold back); an empty slot holds kEmpty, a NaN
@@ -44,6 +51,8 @@ constexpr int kMaxStrips = 32;
 constexpr int kSums = 8; // most sums of one exchange
 constexpr unsigned long long kEmpty = ~0ull;
 constexpr int kMaxPolls = 1 << 18; // about 0.2 s
+// iterations between removals of r's mean (one more sum in that exchange)
+constexpr int kProject = 16;
 
 template <class T>
 using cptr = const __attribute__((address_space(4))) T *;
@@ -574,7 +583,7 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
         {
           const double den = it == 0 ? wr : wr - beta * rr / alpha;
           if (!(den > 0.0))
-            break; // what is left of r lies in the null space
+            break; // r is rounding
           alpha = rr / den;
 #pragma unroll
           for (int k = 0; k < NPT; ++k)
@@ -602,8 +611,33 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
                 v[0] += r[k] * r[k];
                 v[1] += w[k] * r[k];
               }
-          if (!exchange(S2(), v, true, w, h))
+          const bool project = it % kProject == kProject - 1;
+          if (project)
+            {
+              v[2] = 0.0;
+#pragma unroll
+              for (int k = 0; k < NPT; ++k)
+                v[2] += r[k];
+            }
+          if (!(project ? exchange(S3(), v, true, w, h)
+                        : exchange(S2(), v, true, w, h)))
             return give_up();
+          if (project)
+            {
+              // (w and (w, r) do not change: A 1 = 0)
+              const double mean = v[2] / nx;
+              v[0] = fmax(v[0] - mean * v[2], 0.0);
+#pragma unroll
+              for (int k = 0; k < NPT; ++k)
+                {
+                  r[k] -= own[k] ? mean : 0.0;
+                  if (halo[k])
+                    {
+                      rL[q[k]] -= mean;
+                      rL[(nr + 1) * W + q[k]] -= mean;
+                    }
+                }
+            }
           beta = v[0] / rr;
           rr = v[0];
           wr = v[1];

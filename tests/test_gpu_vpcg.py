@@ -69,6 +69,37 @@ def test_potential_matches_oracle(k, nx):
     assert op.solver_stats()[:2] == (it, 2)
 
 
+@pytest.mark.parametrize("k,nx", [(3, [4, 96]), (3, [2, 120]), (3, [50, 18]),
+                                  (2, [2, 300])])
+def test_tolerances_below_rounding(k, nx):
+    """A solve asked for less than b - A phi can reach in 64 bits stays at
+    what it can reach: at most four times the oracle's residual at 1e-12,
+    which is rounding on these meshes (rounding sums in another order: the
+    recurrence restated on the CPU ends at 0.7 to 1.4 times plain CG's)."""
+    print("case: strips, below rounding", k, nx, flush=True)
+    P, mf, f, _ = _pair(k, nx)
+    op = H.VlasovPoissonOperation(mf, poisson_tol=1e-12)
+    fd = torch.empty(P.n_dofs, dtype=torch.float64, device="cuda")
+    for seed in range(4):
+        g = f * (1 + 0.1 * np.random.default_rng(seed).standard_normal(
+            P.n_dofs))
+        fd.copy_(torch.from_numpy(g))
+        b = P.rhs(P.density(g))
+
+        def off(phi):
+            return np.linalg.norm(b - P.poisson_apply(phi)) / \
+                np.linalg.norm(b)
+        bar = 4 * off(P.poisson_solve(b, rel_tol=1e-12)[0])
+        for tol in (3e-13, 1e-13, 1e-15):
+            op.set_poisson_tolerance(tol, 20000)
+            op.set_potential(np.zeros(op.x_n_dofs()))
+            op.update_field(fd)
+            assert off(op.potential()) <= bar, (seed, tol)
+        # and from a start that is already there
+        op.update_field(fd)
+        assert off(op.potential()) <= bar, seed
+
+
 def test_two_operators_in_turn():
     print("case: strips, two operators", flush=True)
     a, b = _pair(3, [8, 8]), _pair(2, [6, 12])
