@@ -858,13 +858,22 @@ size_t sum_slots(const int *n)
 }
 } // namespace vpcg
 
-// Two or more strips whose nodes fit four per thread.
+// Where the strips are the faster solver.  us per iteration, one workgroup and
+// strips, k = 3: 16 x 2 cells 4.9 and 2.7, 32 x 32 11.1 and 3.5; two nodes per
+// thread 64 x 2 4.9 and 4.9, 50 x 18 11.1 and 5.0; four 100 x 2 5.3 and 10.8,
+// 128 x 5 9.3 and 11.6, 100 x 10 11.1 and 11.1.  k = 2: the workgroup holds
+// 512 cells at one per thread, 20 x 20 cells 3.0 and 3.0, 24 x 24 3.6 and
+// 3.0, 32 x 32 5.0 and 3.4; two nodes per thread 60 x 9 3.6 and 4.3.  k = 1:
+// 32 x 32 1.9 and 2.1.
 bool vp_strips_supported(int dim_x, int N, const int *n)
 {
-  if (dim_x != 2 || N < 2 || N > 4 || n[1] < 2)
+  if (dim_x != 2 || n[1] < 2)
     return false;
+  const int T = vpcg::kThreads / (N * N) * (N * N);
   const long long nodes = (long long)vpcg::strip_rows(n[1]) * n[0] * N * N;
-  return nodes <= 4LL * (vpcg::kThreads / (N * N) * (N * N));
+  return N == 4   ? nodes <= 2 * T
+         : N == 3 ? nodes <= T && (long long)n[0] * n[1] > 512
+                  : false;
 }
 
 // 8-byte slots of the inboxes, then the mark
@@ -930,14 +939,10 @@ hipError_t vp_strips_solve(const XDev &xd, int N, const double *rho,
                        st.mark, rel_tol, max_it, stats);
     return hipGetLastError();
   };
-#define HD_STRIP(NN_)                                                        \
-  if (N == NN_)                                                              \
-    return npt <= 1                                                          \
-             ? go(&vpcg::strip_kernel<NN_, 1>, &vpcg::marked_kernel<NN_>)    \
-           : npt <= 2                                                        \
-             ? go(&vpcg::strip_kernel<NN_, 2>, &vpcg::marked_kernel<NN_>)    \
-             : go(&vpcg::strip_kernel<NN_, 4>, &vpcg::marked_kernel<NN_>);
-  HD_STRIP(2) HD_STRIP(3) HD_STRIP(4)
+#define HD_STRIP(NN_, NPT_)                                                  \
+  if (N == NN_ && npt <= NPT_)                                               \
+    return go(&vpcg::strip_kernel<NN_, NPT_>, &vpcg::marked_kernel<NN_>);
+  HD_STRIP(3, 1) HD_STRIP(4, 1) HD_STRIP(4, 2)
 #undef HD_STRIP
   return hipErrorInvalidValue;
 }

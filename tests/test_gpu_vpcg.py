@@ -1,7 +1,7 @@
 """The potential solve on several workgroups (hd_vpcg.hip) against the CPU
 oracle's: strips of one row and of several, an uneven last strip, the fewest
-strips, one, two and four nodes per thread, two operators in turn, and the
-kernel behind a solve that was given up (its mark set from the host; no
+strips, one and two nodes per thread, meshes that stay on one workgroup, two
+operators in turn, and the kernel behind a solve that was given up (its mark set from the host; no
 workgroup waits in that case).
 
 Tolerance: CG to 1e-12 of the right-hand side leaves at most cond(A) 1e-12 in
@@ -23,12 +23,13 @@ L = 4 * np.pi
 MESHES = [
     # degree, x cells
     (3, [5, 2]),      # two strips of one row
-    (1, [7, 6]),
-    (2, [9, 35]),     # two rows per strip, one in the last
+    (1, [7, 6]),      # one workgroup
+    (2, [9, 35]),     # one workgroup
+    (2, [17, 35]),    # two rows per strip, one in the last
     (3, [4, 96]),     # three rows per strip
     (3, [32, 32]),    # the most cells
     (3, [50, 18]),    # two nodes per thread
-    (3, [120, 8]),    # four nodes per thread
+    (3, [120, 8]),    # one workgroup
 ]
 
 
@@ -102,7 +103,7 @@ def test_tolerances_below_rounding(k, nx):
 
 def test_two_operators_in_turn():
     print("case: strips, two operators", flush=True)
-    a, b = _pair(3, [8, 8]), _pair(2, [6, 12])
+    a, b = _pair(3, [8, 8]), _pair(3, [6, 12])
     ops = [H.VlasovPoissonOperation(m[1], poisson_tol=1e-12) for m in (a, b)]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     fs = [torch.from_numpy(m[2]).cuda() for m in (a, b)]
