@@ -13,4 +13,38 @@ int hd_probe_vp_strips(int degree, int n0, int n1)
          hd::vp_strips_supported(2, degree + 1, n);
 }
 
+// The potential solver of a Vlasov-Poisson operator on one workgroup, or on
+// strips with `comm` as their inboxes (hd_probe_strips_bytes of device memory,
+// reset once): the residual image of phi where res_image is given, else a
+// solve from phi, with a guess as x values or (guess_image) as an image.
+// Pointers are the device's; the null stream.
+long long hd_probe_strips_bytes(hd_advection *op)
+{
+  return (long long)hd::vp_strips_bytes(op->mf->nd, op->xdev.n);
+}
+
+int hd_probe_strips_reset(hd_advection *op, void *comm)
+{
+  return (int)hd::vp_strips_reset(comm, op->mf->nd, op->xdev.n);
+}
+
+int hd_probe_poisson(hd_advection *op, void *comm, const double *rho,
+                     double *phi, double *efield, const double *guess,
+                     const float *guess_image, const double *guess_scale,
+                     float *res_image, double *res_scale, double *phi_copy,
+                     double rel_tol, int max_it, long long *stats)
+{
+  hd::ResidualImage residual;
+  residual.image = res_image;
+  residual.scale = res_scale;
+  residual.phi_copy = phi_copy;
+  hd::GuessImage image;
+  image.image = guess_image;
+  image.scale = guess_scale;
+  return (int)hd::vp_poisson(op->xdev, op->mf->nd, rho, phi, guess, efield,
+                             op->work, rel_tol, max_it, stats, nullptr,
+                             op->ptab, res_image ? &residual : nullptr, false,
+                             comm, image);
+}
+
 } // extern "C"

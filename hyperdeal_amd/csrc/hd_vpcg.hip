@@ -31,8 +31,8 @@
 // that the reader sent after it emptied the set (the reader waits for its
 // stores and passes a workgroup barrier before it sends).  A poll is bounded:
 // a workgroup that waits too long (others not scheduled) leaves and marks
-// the solve, which the small kernel launched behind this one then does on
-// its own; without the mark it returns at once.
+// the launch, whose work the small kernel launched behind this one then does
+// on its own; without the mark it returns at once.
 //
 // Measured (MI355X, k = 3): 12 -> 2.7 us per iteration at 32^2 x cells, 4.1 us
 // before the sums went through lane permutations and the stores that empty
@@ -50,7 +50,7 @@ constexpr int kThreads = 512;
 constexpr int kMaxStrips = 32;
 constexpr int kSums = 8; // most sums of one exchange
 constexpr unsigned long long kEmpty = ~0ull;
-constexpr int kMaxPolls = 1 << 18; // about 0.2 s
+constexpr int kMaxPolls = 1 << 18; // about 0.2 s, once per exchange
 // iterations between removals of r's mean (one more sum in that exchange)
 constexpr int kProject = 16;
 
@@ -151,8 +151,7 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
   __shared__ int lost;
   if (t == 0)
     lost = 0;
-  // a residual before this solve gave up: the inboxes are not empty, the
-  // kernel behind does the solve
+  // another workgroup has given up: the kernel behind does the work
   if (*st.mark != 0)
     return;
   // a chain of latencies: its waves go first where a compute unit also works
@@ -248,17 +247,17 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
 #pragma unroll
           for (int k = 0; k < NPT; ++k)
             if (halo[k])
-              fine = receive(st.row_in +
-                               ((par * st.count + sb) * 2 + d) * W + q[k],
-                             h[d][k]) &&
-                     fine;
+              fine = fine && receive(st.row_in +
+                                       ((par * st.count + sb) * 2 + d) * W +
+                                       q[k],
+                                     h[d][k]);
       }
     double a = 0.0;
     if (sums_here)
-      fine = receive(st.sum_in +
+      fine = fine &&
+             receive(st.sum_in +
                        ((par * st.count + sb) * st.count + peer) * kSums + s,
-                     a) &&
-             fine;
+                     a);
     // half a wave holds a sum's terms, one per strip
     if (t < (ns + 1) / 2 * 64)
       {
@@ -494,8 +493,9 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
 #pragma unroll
       for (int k = 0; k < NPT; ++k)
         {
-          x[k] = alpha0 * x[k] + beta0 * g[k];
-          y[k] = alpha0 * y[k] + beta0 * ag[k];
+          // (a guess that is left out may hold NaN)
+          x[k] = beta0 == 0.0 ? alpha0 * x[k] : alpha0 * x[k] + beta0 * g[k];
+          y[k] = beta0 == 0.0 ? alpha0 * y[k] : alpha0 * y[k] + beta0 * ag[k];
         }
     }
   if (res_image)
@@ -704,16 +704,18 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
     }
 }
 
-// The solve behind a marked one: empties the inboxes and runs plain CG from
-// the previous phi (a guess is left out) with its vectors in global memory.
-// One small workgroup with few registers, so that it is scheduled at once
-// beside other work; slow, and only there for correctness.
+// The work behind a marked launch: empties the inboxes and computes the
+// residual image, or runs plain CG from the previous phi (a guess is left out),
+// with its vectors in global memory.  One small workgroup with few registers,
+// so that it is scheduled at once beside other work; slow, and only there for
+// correctness.
 template <int N>
 __global__ __launch_bounds__(256) void marked_kernel(
   XDev xd, const double *__restrict__ tab, const double *__restrict__ rho,
   double *phi, double *__restrict__ efield, double *work,
   unsigned long long *slots, long long n_slots, int *mark, double rel_tol,
-  int max_it, long long *__restrict__ stats)
+  int max_it, long long *__restrict__ stats, float *__restrict__ res_image,
+  double *__restrict__ res_scale, double *__restrict__ phi_copy)
 {
   constexpr int NN = N * N;
   __shared__ double red[256];
@@ -789,6 +791,29 @@ __global__ __launch_bounds__(256) void marked_kernel(
     }
   bb = total(bb);
   rr = total(rr);
+  if (res_image)
+    {
+      s = 0.0;
+      for (int e = threadIdx.x; e < n; e += 256)
+        s += r[e];
+      const double mean = total(s) / n;
+      s = 0.0;
+      for (int e = threadIdx.x; e < n; e += 256)
+        s += (r[e] - mean) * (r[e] - mean);
+      const double rms = sqrt(total(s) / n);
+      const double inv = rms > 0.0 ? 1.0 / rms : 0.0;
+      for (int e = threadIdx.x; e < n; e += 256)
+        {
+          const int c = e / NN, ix = e % N, iy = e % NN / N;
+          res_image[(c / n0 * N + iy) * (n0 * N) + c % n0 * N + ix] =
+            (float)((r[e] - mean) * inv);
+          if (phi_copy)
+            phi_copy[e] = phi[e];
+        }
+      if (threadIdx.x == 0)
+        *res_scale = rms;
+      return;
+    }
   const double rr_start = rr;
   int it = 0;
   while (sqrt(rr) > rel_tol * sqrt(bb) && it < max_it)
@@ -931,12 +956,11 @@ hipError_t vp_strips_solve(const XDev &xd, int N, const double *rho,
                        guess_alone ? 1 : 0, image, scale, copy,
                        guess_image);
     e = hipGetLastError();
-    // (a residual that gives up leaves its mark to the solve that follows)
-    if (e != hipSuccess || residual)
+    if (e != hipSuccess)
       return e;
     hipLaunchKernelGGL(behind, dim3(1), dim3(256), 0, stream, xd, tab2d, rho,
                        phi, efield, work, st.row_in, (long long)slots,
-                       st.mark, rel_tol, max_it, stats);
+                       st.mark, rel_tol, max_it, stats, image, scale, copy);
     return hipGetLastError();
   };
 #define HD_STRIP(NN_, NPT_)                                                  \

@@ -117,69 +117,148 @@ def test_two_operators_in_turn():
         assert _off(op.potential(), m[3]) <= 1e-8
 
 
-class _XDev(ctypes.Structure):
-    _fields_ = [("dim", ctypes.c_int), ("n", ctypes.c_int * 3),
-                ("h", ctypes.c_double * 3), ("n_cells", ctypes.c_longlong),
-                ("kk", ctypes.c_double), ("M", ctypes.c_double * 64),
-                ("K", ctypes.c_double * 64), ("d0", ctypes.c_double * 8),
-                ("d1", ctypes.c_double * 8), ("S", ctypes.c_double * 64),
-                ("G", ctypes.c_double * 64)]
+class _Solver:
+    """The solver of an operator's potential on one workgroup or on strips
+    (hd_probe.hip), with inboxes and statistics of its own."""
+
+    def __init__(self, op):
+        self.op, self.lib = op, ctypes.CDLL(H.library_path())
+        self.lib.hd_probe_strips_bytes.restype = ctypes.c_longlong
+        size = self.lib.hd_probe_strips_bytes(op.handle)
+        self.comm = torch.empty(size // 8, dtype=torch.int64, device="cuda")
+        assert self.lib.hd_probe_strips_reset(op.handle,
+                                              self._p(self.comm)) == 0
+        self.empty()
+        n = op.x_n_dofs()
+        self.phi = torch.zeros(n, dtype=torch.float64, device="cuda")
+        self.field = torch.empty(2 * n, dtype=torch.float64, device="cuda")
+        self.copy = torch.full_like(self.phi, float("nan"))
+        self.scale = torch.empty(1, dtype=torch.float64, device="cuda")
+        self.image = torch.full((n,), float("nan"), dtype=torch.float32,
+                                device="cuda")
+
+    @staticmethod
+    def _p(t):
+        return ctypes.c_void_p(None if t is None else t.data_ptr())
+
+    def empty(self):
+        assert int(self.comm[-1]) == 0 and bool((self.comm[:-1] == -1).all())
+
+    def give_up(self):
+        self.comm[:-1] = 5            # what a broken-off launch may leave
+        self.comm[-1] = 1
+
+    def _call(self, strips, rho, guess, image, scale, residual):
+        stats = torch.zeros(8, dtype=torch.int64, device="cuda")
+        p = self._p
+        out = (self.image, self.scale, self.copy) if residual else [None] * 3
+        torch.cuda.synchronize()
+        rc = self.lib.hd_probe_poisson(
+            self.op.handle, p(self.comm if strips else None), p(rho),
+            p(self.phi), p(self.field), p(guess), p(image), p(scale),
+            *[p(x) for x in out], ctypes.c_double(1e-12), 5000, p(stats))
+        torch.cuda.synchronize()
+        assert rc == 0
+        self.empty()
+        return stats
+
+    def solve(self, rho, strips=True, guess=None, image=None, scale=None):
+        s = self._call(strips, rho, guess, image, scale, False).cpu()
+        return dict(its=int(s[0]), weights=s.view(torch.float64)[6:].numpy(),
+                    start=float(s.view(torch.float64)[3]))
+
+    def residual(self, rho, strips=True):
+        self._call(strips, rho, None, None, None, True)
+        return self.image.cpu().numpy(), float(self.scale)
 
 
 @pytest.mark.parametrize("k,nx", [(3, [6, 5]), (2, [4, 40])])
 def test_marked_solve_runs_on_one_workgroup(k, nx):
     print("case: marked solve", k, nx, flush=True)
     P, mf, f, ref = _pair(k, nx)
-    lib = ctypes.CDLL(H.library_path())
-    N, nc = k + 1, nx[0] * nx[1]
-    t = O.tables(k)
-    S, D, F, w = t["S"], t["D"], t["F"], t["qweights"]
-    G = D @ S
-    x = _XDev(dim=2, n_cells=nc, kk=k * (k + 1.0))
-    x.n[:] = [nx[0], nx[1], 0]
-    x.h[:] = [L / nx[0], 0.8 * L / nx[1], 0.0]
-    for name, m in (("M", S.T @ np.diag(w) @ S), ("K", G.T @ np.diag(w) @ G),
-                    ("S", S), ("G", G), ("d0", F[0] @ G), ("d1", F[1] @ G)):
-        v = np.ascontiguousarray(m).reshape(-1)
-        getattr(x, name)[:len(v)] = list(v)
-    tab = (ctypes.c_double * (8 * N * N))()
-    lib._ZN2hd18vp_poisson2d_tableERKNS_4XDevEiPd(ctypes.byref(x), N, tab)
-    cells = (ctypes.c_int * 3)(nx[0], nx[1], 0)
-    size = lib._ZN2hd15vp_strips_bytesEiPKi
-    size.restype = ctypes.c_size_t
-    n = nc * N * N
-    comm = torch.empty(size(N, cells) // 8, dtype=torch.int64, device="cuda")
-    vp = ctypes.c_void_p
-    assert lib._ZN2hd15vp_strips_resetEPviPKi(vp(comm.data_ptr()), N,
-                                              cells) == 0
-    assert int(comm[-1]) == 0 and bool((comm[:-1] == -1).all())
+    s = _Solver(H.VlasovPoissonOperation(mf, poisson_tol=1e-12))
     rho = torch.from_numpy(P.density(f)).cuda()
-    phi = torch.zeros(n, dtype=torch.float64, device="cuda")
-    work = torch.empty(3 * n, dtype=torch.float64, device="cuda")
-    ef = torch.empty(2 * n, dtype=torch.float64, device="cuda")
-    stats = torch.zeros(8, dtype=torch.int64, device="cuda")
-    tabd = torch.from_numpy(np.array(tab)).cuda()
-    image = (ctypes.c_void_p * 2)()
-    solve = lib._ZN2hd15vp_strips_solveERKNS_4XDevEiPKdPdS4_S5_S5_PvdiPxP12ihipStream_tS4_bPKNS_13ResidualImageERKNS_10GuessImageE  # noqa: E501
 
     def run():
-        rc = solve(ctypes.byref(x), N, vp(rho.data_ptr()), vp(phi.data_ptr()),
-                   None, vp(ef.data_ptr()), vp(work.data_ptr()),
-                   vp(comm.data_ptr()), ctypes.c_double(1e-12), 5000,
-                   vp(stats.data_ptr()), None, vp(tabd.data_ptr()), False,
-                   None, ctypes.byref(image))
-        torch.cuda.synchronize()
-        assert rc == 0
-        assert int(comm[-1]) == 0 and bool((comm[:-1] == -1).all())
-        assert _off(phi.cpu().numpy(), ref) <= 1e-8
-        return int(stats[0]), ef.cpu().numpy()
+        s.phi.zero_()
+        its = s.solve(rho)["its"]
+        assert _off(s.phi.cpu().numpy(), ref) <= 1e-8
+        return its, s.field.cpu().numpy()
 
     its, field = run()
-    phi.zero_()
-    comm[:-1] = 5                 # what a broken-off solve may leave
-    comm[-1] = 1
+    s.give_up()
     its2, field2 = run()
-    assert abs((its2 - its) - its) <= max(3, its // 20)
+    assert abs(its2 - its) <= max(3, its // 20)
     assert np.max(np.abs(field2 - field)) <= 1e-8 * np.max(np.abs(field))
-    phi.zero_()
     run()
+
+
+# one row per strip, an uneven last strip of several rows, two nodes per thread
+IMAGES = [(3, [5, 7]), (2, [17, 35]), (3, [50, 18])]
+
+
+@pytest.mark.parametrize("k,nx", IMAGES)
+def test_residual_image_matches_one_workgroup(k, nx):
+    """The residual image, its scale and the copy of phi: strips, and the
+    kernel behind strips that were given up, against the one-workgroup kernel.
+    Tolerances: b - A phi of a random phi to 1e-13 of its rms (sums of 2 (3 N)
+    products in another order), pixels to that and one FP32 rounding."""
+    print("case: residual image", k, nx, flush=True)
+    P, mf, f, _ = _pair(k, nx)
+    s = _Solver(H.VlasovPoissonOperation(mf, poisson_tol=1e-12))
+    rho = torch.from_numpy(P.density(f)).cuda()
+    phi = np.random.default_rng(k).standard_normal(P.n_x_dofs)
+    s.phi.copy_(torch.from_numpy(phi))
+    ref, scale = s.residual(rho, strips=False)
+    for marked in (False, True, False):
+        s.image.fill_(float("nan"))
+        s.copy.fill_(float("nan"))
+        if marked:
+            s.give_up()
+        img, sc = s.residual(rho)
+        assert abs(sc - scale) <= 1e-12 * scale, marked
+        assert np.max(np.abs(img - ref)) <= 2.5e-7 * np.max(np.abs(ref))
+        assert np.array_equal(s.copy.cpu().numpy(), phi)
+        assert np.array_equal(s.phi.cpu().numpy(), phi)
+
+
+@pytest.mark.parametrize("k,nx", IMAGES)
+def test_guess_image_stands_for_its_dofs(k, nx):
+    """A guess given as an image starts the solve where the same guess given
+    as x values starts it: the weights of phi and the guess and the start's
+    residual agree to 1e-9 (the 2 x 2 system's condition, below 1e4 for random
+    vectors, times rounding of its sums)."""
+    print("case: guess image", k, nx, flush=True)
+    P, mf, f, ref = _pair(k, nx)
+    s = _Solver(H.VlasovPoissonOperation(mf, poisson_tol=1e-12))
+    rho = torch.from_numpy(P.density(f)).cuda()
+    r = np.random.default_rng(k)
+    phi = torch.from_numpy(r.standard_normal(P.n_x_dofs)).cuda()
+    N = k + 1
+    # a part of the solution, so that the guess has a weight
+    img, _ = H.cnn_dofs_to_image(torch.from_numpy(ref).cuda(), nx[0], nx[1], N)
+    img += 0.2 * torch.from_numpy(r.standard_normal(img.shape)).cuda().float()
+    scale = torch.full((1,), 0.75, dtype=torch.float64, device="cuda")
+    dofs = H.cnn_image_to_dofs(img, scale, nx[0], nx[1], N)
+    s.phi.copy_(phi)
+    a = s.solve(rho, guess=dofs)
+    assert abs(a["weights"][1]) > 1e-4
+    s.phi.copy_(phi)
+    b = s.solve(rho, guess=torch.zeros_like(dofs), image=img, scale=scale)
+    np.testing.assert_allclose(b["weights"], a["weights"], rtol=0,
+                               atol=1e-9 * np.abs(a["weights"]).max())
+    assert abs(b["start"] - a["start"]) <= 1e-9 * a["start"]
+    assert _off(s.phi.cpu().numpy(), ref) <= 1e-8
+
+
+def test_nan_guess_is_left_out():
+    print("case: NaN guess", flush=True)
+    P, mf, f, ref = _pair(3, [8, 6])
+    s = _Solver(H.VlasovPoissonOperation(mf, poisson_tol=1e-12))
+    rho = torch.from_numpy(P.density(f)).cuda()
+    plain = s.solve(rho)
+    for bad in (float("nan"), float("inf")):
+        s.phi.zero_()
+        r = s.solve(rho, guess=torch.full_like(s.phi, bad))
+        assert list(r["weights"]) == [1.0, 0.0] and r["its"] == plain["its"]
+        assert _off(s.phi.cpu().numpy(), ref) <= 1e-8
