@@ -247,12 +247,8 @@ cv_block(T *lds, const T *__restrict__ src, T *__restrict__ dst,
       wave_sync();
       // the solution (LSRK stage), used at the end
       double ps[KU];
-      if constexpr (MODE == 1)
-        {
-          // (FP64: a stage whose input is the solution has it in B1)
-          if (sizeof(T) == 4 || stage.keep != kSolInput)
-            for_values(n_in, [&](int k, int e) { ps[k] = stage.sol[base + e]; });
-        }
+      if constexpr (MODE != 0 && MODE != 3)
+        for_values(n_in, [&](int k, int e) { ps[k] = stage.sol[base + e]; });
       // V: K = P + sum over v0, v1, along the lines of this lane's v-plane
       if (busy)
         {
@@ -308,16 +304,18 @@ cv_block(T *lds, const T *__restrict__ src, T *__restrict__ dst,
           dst[base + e] = a;
         else
           {
-            double so = ps[k];
-            if constexpr (sizeof(T) == 8)
-              {
-                const double own = lds[lofs(k) + N2 * P];
-                so = stage.keep == kSolInput ? own
-                                             : stage_solution(stage, so, own);
-              }
-            if (sizeof(T) == 4 || stage.keep == kSolUpdate)
+            // (the input's own values are in B1)
+            double so;
+            if constexpr (MODE == 3)
+              so = (double)lds[lofs(k) + N2 * P];
+            else if constexpr (MODE == 5)
+              so = ps[k] +
+                   stage.recover * ((double)lds[lofs(k) + N2 * P] - ps[k]);
+            else
+              so = ps[k];
+            if constexpr (MODE == 1 || MODE == 5)
               stage.sol[base + e] = so + stage.b_dt * (double)a;
-            if (stage.ti_out)
+            if (MODE == 3 || MODE == 4 || stage.ti_out)
               static_cast<T *>(stage.ti_out)[base + e] =
                 (T)(so + stage.a_dt * (double)a);
           }
@@ -371,20 +369,26 @@ hipError_t launch(int mode, const T *src, T *dst, const T *coef,
                             dev) != hipSuccess ||
       cus < 8)
     cus = 256;
-  const int wpc =
-    mode == 0 ? waves_per_cu<N, T, 0>() : waves_per_cu<N, T, 1>();
-  long long grid = (long long)cus * wpc;
-  grid = std::min<long long>(grid, (n_groups + 7) / 8 * 8);
-  grid = std::max<long long>(8, grid / 8 * 8);
+  auto go = [&](auto kernel, int wpc) {
+    long long grid = (long long)cus * wpc;
+    grid = std::min<long long>(grid, (n_groups + 7) / 8 * 8);
+    grid = std::max<long long>(8, grid / 8 * 8);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64), 0, stream, src,
+                       dst, coef, mesh, inflow, stage, n_groups);
+    return hipGetLastError();
+  };
   if (mode == 0)
-    hipLaunchKernelGGL((cv_kernel<N, T, 0>), dim3((unsigned)grid), dim3(64),
-                       0, stream, src, dst, coef, mesh, inflow, stage,
-                       n_groups);
-  else
-    hipLaunchKernelGGL((cv_kernel<N, T, 1>), dim3((unsigned)grid), dim3(64),
-                       0, stream, src, dst, coef, mesh, inflow, stage,
-                       n_groups);
-  return hipGetLastError();
+    return go(cv_kernel<N, T, 0>, waves_per_cu<N, T, 0>());
+  if constexpr (sizeof(T) == 8)
+    {
+      if (stage.keep == kSolInput)
+        return go(cv_kernel<N, T, 3>, waves_per_cu<N, T, 3>());
+      if (stage.keep == kSolKeep)
+        return go(cv_kernel<N, T, 4>, waves_per_cu<N, T, 4>());
+      if (stage.recover != 0.0)
+        return go(cv_kernel<N, T, 5>, waves_per_cu<N, T, 5>());
+    }
+  return go(cv_kernel<N, T, 1>, waves_per_cu<N, T, 1>());
 }
 
 template <typename T>
@@ -449,10 +453,9 @@ __global__ __launch_bounds__(64) void batch_kernel(
       stage.a_dt = ptrs.a_dt;
       stage.b_dt = ptrs.b_dt;
       stage.recover = ptrs.recover;
-      stage.keep = ptrs.keep;
       stage.sol = MODE == 0 ? nullptr : ptrs.sol[tk.op];
-      stage.ti_out = MODE == 1 ? ptrs.ti[tk.op] : nullptr;
-      cv_block<N, T, MODE == 0 ? 0 : 1>(
+      stage.ti_out = MODE == 0 || MODE == 2 ? nullptr : ptrs.ti[tk.op];
+      cv_block<N, T, MODE == 2 ? 1 : MODE>(
         lds, static_cast<const T *>(ptrs.src[tk.op]),
         MODE == 0 ? static_cast<T *>(ptrs.dst[tk.op]) : nullptr,
         static_cast<const T *>(o.coef), mesh, inflow, stage, tk.lb, tk.le,
@@ -472,8 +475,23 @@ hipError_t batch_launch(int mode, const BatchOp *ops, const BatchTask *tasks,
                        tasks, plan, ptrs);
   };
   if (mode == 0)
-    go(batch_kernel<N, T, 0>);
-  else if (mode == 1)
+    {
+      go(batch_kernel<N, T, 0>);
+      return hipGetLastError();
+    }
+  if constexpr (sizeof(T) == 8)
+    {
+      // (ptrs.ti is null in a last stage)
+      if (ptrs.keep == kSolInput)
+        go(batch_kernel<N, T, 3>);
+      else if (ptrs.keep == kSolKeep)
+        go(batch_kernel<N, T, 4>);
+      else if (ptrs.recover != 0.0)
+        go(batch_kernel<N, T, 5>);
+      if (ptrs.keep != kSolUpdate || ptrs.recover != 0.0)
+        return hipGetLastError();
+    }
+  if (mode == 1)
     go(batch_kernel<N, T, 1>);
   else
     go(batch_kernel<N, T, 2>);
