@@ -110,6 +110,16 @@ int vp_update(hd_advection *op, const double *f, const float *f32,
   return e == hipSuccess ? HD_OK : hip_fail(e, "Vlasov-Poisson field update");
 }
 
+// the factorised form of a periodic deformed operator serves this call (if its
+// vectors are 16-byte aligned)
+bool curved_active(const hd_advection *op, int mode, int precision)
+{
+  const hd_matrix_free *mf = op->mf;
+  return op->has_curved && op->algorithm == HD_ALGO_AUTO &&
+         hd::curved_faster(mf->dim_x, mf->dim_v, mf->nd, mf->mesh.n_cells,
+                           precision == HD_FP64, mode != 0);
+}
+
 // density: where a Vlasov-Poisson operator takes rho from (VpDensity);
 // sol: the FP64 solution (kDensitySolution)
 int run_operator(hd_advection *op, int mode, int precision, const void *src,
@@ -268,7 +278,7 @@ int run_operator(hd_advection *op, int mode, int precision, const void *src,
                   static_cast<float *>(dst), op->coef32, mf->mesh, op->inflow,
                   op->quad, stage, time, mf->dim_x, stream);
     }
-  else if (op->has_curved && op->algorithm == HD_ALGO_AUTO &&
+  else if (curved_active(op, mode, precision) &&
            (reinterpret_cast<uintptr_t>(src) |
             reinterpret_cast<uintptr_t>(dst)) %
                16 ==
@@ -324,7 +334,7 @@ bool defers_solution(const hd_advection *op, const double *sol,
   if (op->vp)
     return false;
   return choose_algorithm(op, HD_FP64) == HD_ALGO_COLLAPSED ||
-         (op->has_curved && op->algorithm == HD_ALGO_AUTO);
+         curved_active(op, 1, HD_FP64);
 }
 
 bool valid_precision(int p) { return p == HD_FP64 || p == HD_FP32; }
@@ -684,9 +694,15 @@ int hd_advection_create(hd_matrix_free *mf, const double *velocity,
       op->geo.xfg = parts[1];
       op->geo.vca = parts[2];
       op->geo.vfg = parts[3];
-      if (all_periodic && hd::curved_supported(mf->dim_x, mf->dim_v, nd,
-                                               mf->xmap.n_cells(),
-                                               mf->vmap.n_cells()))
+      const auto faster = [&](bool fp64, bool stage) {
+        return hd::curved_faster(mf->dim_x, mf->dim_v, nd, mf->mesh.n_cells,
+                                 fp64, stage);
+      };
+      if (all_periodic &&
+          hd::curved_supported(mf->dim_x, mf->dim_v, nd, mf->xmap.n_cells(),
+                               mf->vmap.n_cells()) &&
+          (faster(true, false) || faster(true, true) ||
+           faster(false, false) || faster(false, true)))
         {
           hd::CurvedHost hx, hv;
           hd::curved_space_operator(mf->xmap, t, skew_factor, xc, xf, hx);

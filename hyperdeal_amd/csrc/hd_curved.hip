@@ -605,6 +605,38 @@ bool curved_supported(int dim_x, int dim_v, int N, long long n_x_cells,
   return true;
 }
 
+// Where this form is faster than the quadrature kernel.  Up to 50,000 cells it
+// always is: the other one is bound by latency there (1+1, k = 1 apply 18 us
+// from the smallest to 220^2 cells, here 8 to 17).  Above, tiles of 16 x 16
+// that a cell of 2 x 2 values leaves empty cost more than the other kernel's
+// passes, and a stage's accesses, element by element where nodes do not fill a
+// tile, cost more than its arithmetic saves.  us for this form and the other,
+// 1+1 FP64 steps: k = 1 270^2 cells 121 and 114, k = 2 800^2 956 and 952, k = 4
+// 500^2 671 and 792, 1100^2 3837 and 3673; FP32 steps: k = 2 270^2 146 and 173,
+// 330^2 210 and 182, k = 3 270^2 174 and 177, 420^2 440 and 324, k = 4 500^2
+// 690 and 704, 800^2 1635 and 1602; FP32 apply k = 2 800^2 122 and 125, 1100^2
+// 226 and 217.  k = 1 FP32 steps: 2+1 40^3 166 and 245, 50^3 302 and 286; 1+2
+// 100^3 1505 and 1518, 140^3 4551 and 4096.  All else: faster throughout.
+bool curved_faster(int dim_x, int dim_v, int N, long long cells, bool fp64,
+                   bool stage)
+{
+  if (cells <= 50000)
+    return true;
+  if (dim_x + dim_v == 2)
+    {
+      if (N == 2)
+        return false;
+      if (!stage)
+        return fp64 || N > 3 || cells <= 600000;
+      if (fp64)
+        return N == 4 || cells <= 500000;
+      return cells <= (N == 5 ? 250000 : 75000);
+    }
+  if (dim_x + dim_v == 3 && N == 2 && stage && !fp64)
+    return cells <= (dim_x == 1 ? 1000000 : 100000);
+  return true;
+}
+
 hipError_t curved_create(int dim_x, int dim_v, int N, const CurvedHost &x,
                          const CurvedHost &v, CurvedDev *out)
 {

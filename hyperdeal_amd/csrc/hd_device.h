@@ -366,6 +366,8 @@ struct CurvedDev
 struct CurvedHost;
 bool curved_supported(int dim_x, int dim_v, int N, long long n_x_cells,
                       long long n_v_cells);
+bool curved_faster(int dim_x, int dim_v, int N, long long cells, bool fp64,
+                   bool stage);
 hipError_t curved_create(int dim_x, int dim_v, int N, const CurvedHost &x,
                          const CurvedHost &v, CurvedDev *out);
 void curved_destroy(CurvedDev &c);

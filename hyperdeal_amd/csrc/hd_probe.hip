@@ -13,6 +13,16 @@ int hd_probe_vp_strips(int degree, int n0, int n1)
          hd::vp_strips_supported(2, degree + 1, n);
 }
 
+// 1: an apply or stage on a periodic deformed mesh takes the factorised form;
+// x_cells and v_cells: of the two spaces
+int hd_probe_curved(int dim_x, int dim_v, int degree, long long x_cells,
+                    long long v_cells, int precision, int stage)
+{
+  return hd::curved_supported(dim_x, dim_v, degree + 1, x_cells, v_cells) &&
+         hd::curved_faster(dim_x, dim_v, degree + 1, x_cells * v_cells,
+                           precision == HD_FP64, stage != 0);
+}
+
 // The potential solver of a Vlasov-Poisson operator on one workgroup, or on
 // strips with `comm` as their inboxes (hd_probe_strips_bytes of device memory,
 // reset once): the residual image of phi where res_image is given, else a

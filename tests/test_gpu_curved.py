@@ -89,9 +89,48 @@ def test_matches_oracle(dims, k, n, skew, nq, coll):
                                      (s0 + 0.3 * r))) <= scale + ulp
 
 
-def test_large_meshes_and_three_dimensions_take_the_quadrature_kernel():
-    P, mf, op = _pair((3, 1), 2, [2, 2, 3, 4], 0.0, None, False, seed=8)
+@pytest.mark.parametrize("dims,k,n,curved", [
+    ((3, 1), 2, [2, 2, 3, 4], False),
+    ((1, 1), 1, [270, 270], False),      # tiles mostly empty, many cells
+    ((2, 1), 4, [73, 74, 2], True),      # 5,402 x cells
+    ((2, 1), 4, [74, 74, 2], False),     # tables of one space above 64 MB
+])
+def test_other_meshes_take_the_quadrature_kernel(dims, k, n, curved):
+    print("case: curved or quadrature", dims, k, n, flush=True)
+    P, mf, op = _pair(dims, k, n, 0.0, None, False, seed=8)
+    src = torch.from_numpy(np.random.default_rng(3).standard_normal(
+        P.n_dofs)).cuda()
+    auto = op.apply(torch.empty_like(src), src).cpu().numpy()
+    op.set_algorithm(H.ALGO_QUADRATURE)
+    quad = op.apply(torch.empty_like(src), src).cpu().numpy()
+    assert _rel(auto, quad) <= 1e-12
+    assert np.array_equal(auto, quad) != curved
+
+
+@pytest.mark.parametrize("dims,k,n,zero", [
+    ((1, 1), 3, [5, 6], [0]), ((1, 1), 2, [4, 7], [0, 1]),
+    ((2, 2), 3, [3, 2, 2, 3], [0, 1]), ((2, 2), 2, [3, 4, 2, 3], [2, 3]),
+    ((2, 2), 1, [3, 2, 3, 2], [1, 2]), ((2, 1), 4, [3, 2, 3], [0, 2]),
+])
+def test_zero_velocities(dims, k, n, zero):
+    """Directions, or a whole space, that nothing flows along: their faces
+    carry nothing and are skipped."""
+    print("case: curved, zero velocities", dims, k, n, zero, flush=True)
+    D = sum(dims)
+    a = np.random.default_rng(k).uniform(0.2, 1, D)
+    a[1::2] *= -1
+    a[zero] = 0
+    lo, hi = [-1.0] * D, [1.0] * D
+    P = O.Problem(dims[0], dims[1], k, n, lo, hi, list(a))
+    P.set_deformation(0.1, 2)
+    mf = H.MatrixFree(dims[0], dims[1], k, n, lo, hi)
+    mf.set_deformation(0.1, 2)
+    op = H.AdvectionOperation(mf, list(a))
     u = np.random.default_rng(3).standard_normal(P.n_dofs)
+    ref = P.apply(u)
     src = torch.from_numpy(u).cuda()
-    dst = op.apply(torch.empty_like(src), src)
-    assert _rel(dst.cpu().numpy(), P.apply(u)) <= 1e-12
+    for prec, x, tol in ((H.FP64, src, 1e-12), (H.FP32, src.float(), 2e-6)):
+        dst = op.apply(torch.empty_like(x), x, precision=prec)
+        err = np.abs(dst.double().cpu().numpy() - P.apply(
+            x.double().cpu().numpy()))
+        assert err.max() <= tol * max(np.abs(ref).max(), 1.0)
