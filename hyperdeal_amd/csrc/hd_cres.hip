@@ -82,7 +82,7 @@ struct Geo<5, float>
   static constexpr int HALVES = 1, BLOCK = 256, WAVES = 3;
 };
 
-template <int N, class T, int MODE>
+template <int N, class T, int MODE, int HALVES>
 __global__ __launch_bounds__((Geo<N, T>::BLOCK), (Geo<N, T>::WAVES)) void
   cres_kernel(const T *__restrict__ src_, T *__restrict__ dst_,
               const T *__restrict__ coef, MeshDev mesh, InflowDev inflow,
@@ -110,9 +110,9 @@ __global__ __launch_bounds__((Geo<N, T>::BLOCK), (Geo<N, T>::WAVES)) void
   // consecutive cells per XCD (blocks are dispatched round-robin over them);
   // HALVES blocks share a cell: block h keeps the planes i5 = h, h + HALVES,
   // .. and takes the other planes of the input for direction 5 only, from
-  // the L2 that the other block's loads have filled (step is even, so h is
-  // the block's own)
-  constexpr int HALVES = G::HALVES, NPL = (N + HALVES - 1) / HALVES;
+  // the L2 that the other blocks' loads have filled (step is a multiple of
+  // HALVES, so h is the block's own)
+  constexpr int NPL = (N + HALVES - 1) / HALVES;
   static_assert(N % HALVES == 0, "planes per block");
   const long long per = (mesh.n_cells + 7) / 8 * HALVES;
   const long long u_end =
@@ -352,33 +352,54 @@ hipError_t launch(int mode, const T *src, T *dst, const T *coef,
                             dev) != hipSuccess ||
       cus < 8)
     cus = 256;
-  auto go = [&](auto kernel) {
-    // as many persistent blocks as are resident, a multiple of the XCDs
+  // as many persistent blocks as are resident, a multiple of the XCDs
+  auto resident = [&](auto kernel) {
     int bpc = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, kernel, G::BLOCK,
                                                      0) != hipSuccess ||
         bpc < 1)
       bpc = 1;
-    const long long most = (mesh.n_cells + 7) / 8 * 8 * G::HALVES;
+    return (long long)cus * bpc;
+  };
+  auto start = [&](auto kernel, int halves, long long blocks) {
+    const long long most = (mesh.n_cells + 7) / 8 * 8 * halves;
     const unsigned grid = (unsigned)std::min<long long>(
-      most, (long long)(cus * bpc) / (8 * G::HALVES) * (8 * G::HALVES));
+      most, blocks / (8 * halves) * (8 * halves));
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(G::BLOCK), 0, stream, src,
                        dst, coef, mesh, inflow, stage);
     return hipGetLastError();
   };
+  // Few cells: a block per output plane, as long as all are resident at once
+  // (a cell's N chunks one after the other are what a small mesh waits for).
+  // us for an apply, the two-pass split form, a cell per block (k = 5 FP64: two
+  // blocks) and a plane per block: k = 4 FP64 1 cell 17, 32, 12, 96 cells 28,
+  // 33, 16; k = 4 FP32 1 cell -, 24, 9.5; k = 5 FP64 1 cell 25, 31, 19, 16 cells
+  // 28, 32, 20; k = 5 FP32 1 cell -, 36, 13.  With more cells than that a plane
+  // per block reads every input value N times from L2.
+  auto go = [&](auto mode_c) {
+    constexpr int MODE = decltype(mode_c)::value;
+    const auto planes = cres_kernel<N, T, MODE, N>;
+    const long long blocks = resident(planes);
+    if (mesh.n_cells * N <= blocks)
+      return start(planes, N, blocks);
+    const auto cells = cres_kernel<N, T, MODE, G::HALVES>;
+    return start(cells, G::HALVES, resident(cells));
+  };
+  using std::integral_constant;
   if (mode == 0)
-    return go(cres_kernel<N, T, 0>);
+    return go(integral_constant<int, 0>());
   if constexpr (sizeof(T) == 8)
     {
       if (stage.keep == kSolInput)
-        return go(cres_kernel<N, T, 3>);
+        return go(integral_constant<int, 3>());
       if (stage.keep == kSolKeep)
-        return go(cres_kernel<N, T, 4>);
+        return go(integral_constant<int, 4>());
       if (stage.recover != 0.0)
-        return stage.ti_out ? go(cres_kernel<N, T, 5>)
-                            : go(cres_kernel<N, T, 6>);
+        return stage.ti_out ? go(integral_constant<int, 5>())
+                            : go(integral_constant<int, 6>());
     }
-  return stage.ti_out ? go(cres_kernel<N, T, 1>) : go(cres_kernel<N, T, 2>);
+  return stage.ti_out ? go(integral_constant<int, 1>())
+                      : go(integral_constant<int, 2>());
 }
 } // namespace cres
 

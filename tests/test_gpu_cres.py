@@ -19,6 +19,10 @@ FORMS = [
     # degree, cells, velocity (both signs, one direction without transport)
     (5, [3, 3, 2, 3, 3, 2], [0.7, -0.4, 0.5, 0.0, -0.9, 0.55]),
     (4, [3, 4, 3, 3, 3, 3], [-0.6, 0.2, -0.8, 0.35, 0.5, -0.7]),
+    # few cells: a block per output plane
+    (5, [2, 1, 2, 1, 2, 1], [0.7, -0.4, 0.5, 0.3, -0.9, 0.55]),
+    (4, [1, 2, 3, 1, 2, 1], [-0.6, 0.2, -0.8, 0.35, 0.0, -0.7]),
+    (4, [3, 2, 2, 2, 2, 2], [0.6, 0.2, 0.8, -0.35, 0.5, 0.7]),
 ]
 
 
