@@ -255,6 +255,18 @@ __device__ inline void tile_read(const T *buf, int base, T *u)
     }
 }
 
+// row rb of the tile
+template <int D, int N, typename T, int p>
+__device__ inline void row_read(const T *buf, int base, int rb, T *u)
+{
+  using PL = Plan<D, N>;
+  const volatile __attribute__((address_space(3))) T *vb =
+    (const volatile __attribute__((address_space(3))) T *)buf;
+#pragma unroll
+  for (int r = 0; r < N; ++r)
+    u[r] = vb[base + r * PL::W(PL::a(p)) + rb * PL::W(PL::b(p))];
+}
+
 template <int D, int N, typename T, int p>
 __device__ inline void tile_write(T *buf, int base, const T *u)
 {
@@ -737,9 +749,6 @@ apply_block(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ src_,
         face_load<D, N, T, p>(src, gbase[p], nnb, fnode, fc[p]);
         if (store)
           {
-            // (large tiles read the input's values again from U)
-            if constexpr (kLateLast && (MODE == 3 || MODE == 5 || MODE == 6))
-              tile_read<D, N, T, p>(U, lbase[p], ul);
             if constexpr (kReadsSol && !kEarlySol)
               {
 #pragma unroll
@@ -747,6 +756,26 @@ apply_block(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ src_,
                   sv[r] =
                     sol[g0 + (r % N) * ipow(N, a) + (r / N) * ipow(N, b)];
               }
+            // FP64: the input's own values are at hand for a solution that
+            // the previous stage left (large tiles read them again from U,
+            // a row at a time: the whole tile spills)
+            if constexpr (MODE == 5 || MODE == 6)
+              {
+#pragma unroll
+                for (int rb = 0; rb < N; ++rb)
+                  {
+                    if constexpr (kLateLast)
+                      {
+                        row_read<D, N, T, p>(U, lbase[p], rb, ul + N * rb);
+                        __builtin_amdgcn_sched_barrier(0);
+                      }
+#pragma unroll
+                    for (int r = N * rb; r < N * rb + N; ++r)
+                      sv[r] += stage.recover * ((double)ul[r] - sv[r]);
+                  }
+              }
+            if constexpr (kLateLast && MODE == 3)
+              tile_read<D, N, T, p>(U, lbase[p], ul);
 #pragma unroll
             for (int r = 0; r < NN; ++r)
               {
@@ -756,13 +785,9 @@ apply_block(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ src_,
                   __builtin_nontemporal_store(out[r], &dst[g]);
                 else
                   {
-                    // FP64: the input's own values are at hand for a
-                    // solution that the previous stage left
                     double s;
                     if constexpr (MODE == 3)
                       s = (double)ul[r];
-                    else if constexpr (MODE == 5 || MODE == 6)
-                      s = sv[r] + stage.recover * ((double)ul[r] - sv[r]);
                     else
                       s = sv[r];
                     if constexpr (kWritesSol)
