@@ -51,8 +51,11 @@ constexpr int kMaxStrips = 32;
 constexpr int kSums = 8; // most sums of one exchange
 constexpr unsigned long long kEmpty = ~0ull;
 constexpr int kMaxPolls = 1 << 18; // about 0.2 s, once per exchange
-// iterations between removals of r's mean (one more sum in that exchange)
-constexpr int kProject = 16;
+// iterations between removals of r's mean (one more exchange; restated on the
+// CPU, every iteration to every 64th end at the same residuals.  As a third sum
+// of every 16th exchange it cost every iteration 8 %, 3.13 -> 3.38 us at 32^2
+// cells)
+constexpr int kProject = 64;
 
 template <class T>
 using cptr = const __attribute__((address_space(4))) T *;
@@ -579,69 +582,71 @@ __global__ __launch_bounds__(kThreads) void strip_kernel(
       if (!exchange(S1(), v, true, w, h))
         return give_up();
       double wr = v[0], alpha = 0.0, beta = 0.0;
-      while (sqrt(rr) > stop && it < max_it)
+      bool go = true;
+      while (go && sqrt(rr) > stop && it < max_it)
         {
-          const double den = it == 0 ? wr : wr - beta * rr / alpha;
-          if (!(den > 0.0))
-            break; // r is rounding
-          alpha = rr / den;
-#pragma unroll
-          for (int k = 0; k < NPT; ++k)
+          const int until = min(max_it, it + kProject);
+          while (sqrt(rr) > stop && it < until)
             {
-              p[k] = r[k] + beta * p[k];
-              s[k] = w[k] + beta * s[k];
-              x[k] += alpha * p[k];
-              r[k] -= alpha * s[k];
-              if (halo[k])
-                {
-                  sh[0][k] = h[0][k] + beta * sh[0][k];
-                  sh[1][k] = h[1][k] + beta * sh[1][k];
-                  rL[q[k]] -= alpha * sh[0][k];
-                  rL[(nr + 1) * W + q[k]] -= alpha * sh[1][k];
-                }
-            }
-          store_r();
-          lds_barrier();
-          product(w);
-          v[0] = v[1] = 0.0;
-#pragma unroll
-          for (int k = 0; k < NPT; ++k)
-            if (own[k])
-              {
-                v[0] += r[k] * r[k];
-                v[1] += w[k] * r[k];
-              }
-          const bool project = it % kProject == kProject - 1;
-          if (project)
-            {
-              v[2] = 0.0;
-#pragma unroll
-              for (int k = 0; k < NPT; ++k)
-                v[2] += r[k];
-            }
-          if (!(project ? exchange(S3(), v, true, w, h)
-                        : exchange(S2(), v, true, w, h)))
-            return give_up();
-          if (project)
-            {
-              // (w and (w, r) do not change: A 1 = 0)
-              const double mean = v[2] / nx;
-              v[0] = fmax(v[0] - mean * v[2], 0.0);
+              const double den = it == 0 ? wr : wr - beta * rr / alpha;
+              go = den > 0.0;
+              if (!go)
+                break; // r is rounding
+              alpha = rr / den;
 #pragma unroll
               for (int k = 0; k < NPT; ++k)
                 {
-                  r[k] -= own[k] ? mean : 0.0;
+                  p[k] = r[k] + beta * p[k];
+                  s[k] = w[k] + beta * s[k];
+                  x[k] += alpha * p[k];
+                  r[k] -= alpha * s[k];
                   if (halo[k])
                     {
-                      rL[q[k]] -= mean;
-                      rL[(nr + 1) * W + q[k]] -= mean;
+                      sh[0][k] = h[0][k] + beta * sh[0][k];
+                      sh[1][k] = h[1][k] + beta * sh[1][k];
+                      rL[q[k]] -= alpha * sh[0][k];
+                      rL[(nr + 1) * W + q[k]] -= alpha * sh[1][k];
                     }
                 }
+              store_r();
+              lds_barrier();
+              product(w);
+              v[0] = v[1] = 0.0;
+#pragma unroll
+              for (int k = 0; k < NPT; ++k)
+                if (own[k])
+                  {
+                    v[0] += r[k] * r[k];
+                    v[1] += w[k] * r[k];
+                  }
+              if (!exchange(S2(), v, true, w, h))
+                return give_up();
+              beta = v[0] / rr;
+              rr = v[0];
+              wr = v[1];
+              ++it;
             }
-          beta = v[0] / rr;
-          rr = v[0];
-          wr = v[1];
-          ++it;
+          if (!go || it < until || it == max_it)
+            break;
+          // r's mean, in the own rows and the copies of the neighbours' (w
+          // and (w, r) do not change: A 1 = 0)
+          v[0] = 0.0;
+#pragma unroll
+          for (int k = 0; k < NPT; ++k)
+            v[0] += r[k];
+          if (!exchange(S1(), v, false, r, h))
+            return give_up();
+          const double mean = v[0] / nx;
+#pragma unroll
+          for (int k = 0; k < NPT; ++k)
+            {
+              r[k] -= own[k] ? mean : 0.0;
+              if (halo[k])
+                {
+                  rL[q[k]] -= mean;
+                  rL[(nr + 1) * W + q[k]] -= mean;
+                }
+            }
         }
     }
 
@@ -883,21 +888,22 @@ size_t sum_slots(const int *n)
 }
 } // namespace vpcg
 
-// Where the strips are the faster solver.  us per iteration, one workgroup and
-// strips, k = 3: 16 x 2 cells 4.9 and 2.7, 32 x 32 11.1 and 3.5; two nodes per
-// thread 64 x 2 4.9 and 4.9, 50 x 18 11.1 and 5.0; four 100 x 2 5.3 and 10.8,
-// 128 x 5 9.3 and 11.6, 100 x 10 11.1 and 11.1.  k = 2: the workgroup holds
-// 512 cells at one per thread, 20 x 20 cells 3.0 and 3.0, 24 x 24 3.6 and
-// 3.0, 32 x 32 5.0 and 3.4; two nodes per thread 60 x 9 3.6 and 4.3.  k = 1:
-// 32 x 32 1.9 and 2.1.
+// Where the strips are the faster solver: one workgroup holds 512 cells at one
+// per thread.  us per iteration, one workgroup and strips, k = 3: 16 x 2 cells
+// 4.9 and 2.7, 32 x 32 11.0 and 3.1; two nodes per thread 64 x 2 4.9 and 4.9,
+// 50 x 18 11.0 and 4.6; four 128 x 2 5.2 and 8.7, 128 x 5 9.2 and 8.9, 100 x 10
+// 11.0 and 8.3, 66 x 9 9.2 and 6.7.  k = 2: 20 x 20 cells 3.0 and 3.0, 24 x 24
+// 3.6 and 3.0, 32 x 32 5.0 and 3.1; two nodes per thread 60 x 9 3.6 and 4.3.
+// k = 1: 32 x 32 1.9 and 2.1.
 bool vp_strips_supported(int dim_x, int N, const int *n)
 {
   if (dim_x != 2 || n[1] < 2)
     return false;
   const int T = vpcg::kThreads / (N * N) * (N * N);
   const long long nodes = (long long)vpcg::strip_rows(n[1]) * n[0] * N * N;
-  return N == 4   ? nodes <= 2 * T
-         : N == 3 ? nodes <= T && (long long)n[0] * n[1] > 512
+  const bool two = (long long)n[0] * n[1] > 512;
+  return N == 4   ? nodes <= (two ? 4 : 2) * T
+         : N == 3 ? two && nodes <= T
                   : false;
 }
 
@@ -966,7 +972,7 @@ hipError_t vp_strips_solve(const XDev &xd, int N, const double *rho,
 #define HD_STRIP(NN_, NPT_)                                                  \
   if (N == NN_ && npt <= NPT_)                                               \
     return go(&vpcg::strip_kernel<NN_, NPT_>, &vpcg::marked_kernel<NN_>);
-  HD_STRIP(3, 1) HD_STRIP(4, 1) HD_STRIP(4, 2)
+  HD_STRIP(3, 1) HD_STRIP(4, 1) HD_STRIP(4, 2) HD_STRIP(4, 4)
 #undef HD_STRIP
   return hipErrorInvalidValue;
 }

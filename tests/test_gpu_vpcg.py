@@ -1,6 +1,6 @@
 """The potential solve on several workgroups (hd_vpcg.hip) against the CPU
 oracle's: strips of one row and of several, an uneven last strip, the fewest
-strips, one and two nodes per thread, meshes that stay on one workgroup, two
+strips, one, two and four nodes per thread, meshes that stay on one workgroup, two
 operators in turn, and the kernel behind a solve that was given up (its mark set from the host; no
 workgroup waits in that case).
 
@@ -29,7 +29,7 @@ MESHES = [
     (3, [4, 96]),     # three rows per strip
     (3, [32, 32]),    # the most cells
     (3, [50, 18]),    # two nodes per thread
-    (3, [120, 8]),    # one workgroup
+    (3, [120, 8]),    # four nodes per thread
 ]
 
 
@@ -70,7 +70,7 @@ def test_potential_matches_oracle(k, nx):
     assert op.solver_stats()[:2] == (it, 2)
 
 
-@pytest.mark.parametrize("k,nx", [(3, [4, 96]), (3, [2, 120]), (3, [50, 18]),
+@pytest.mark.parametrize("k,nx", [(3, [4, 96]), (3, [2, 120]), (3, [120, 8]),
                                   (2, [2, 300])])
 def test_tolerances_below_rounding(k, nx):
     """A solve asked for less than b - A phi can reach in 64 bits stays at
@@ -193,8 +193,9 @@ def test_marked_solve_runs_on_one_workgroup(k, nx):
     run()
 
 
-# one row per strip, an uneven last strip of several rows, two nodes per thread
-IMAGES = [(3, [5, 7]), (2, [17, 35]), (3, [50, 18])]
+# one row per strip, an uneven last strip of several rows, two and four nodes
+# per thread
+IMAGES = [(3, [5, 7]), (2, [17, 35]), (3, [50, 18]), (3, [120, 8])]
 
 
 @pytest.mark.parametrize("k,nx", IMAGES)

@@ -15,7 +15,7 @@ def _lib():
 @pytest.mark.parametrize("k,nx,strips", [
     (3, [16, 2], 1), (3, [2, 2], 1), (3, [32, 32], 1), (3, [4, 256], 1),
     (3, [64, 2], 1), (3, [64, 16], 1), (3, [65, 2], 0), (3, [100, 2], 0),
-    (3, [128, 5], 0), (3, [5, 1], 0),
+    (3, [128, 4], 0), (3, [128, 5], 1), (3, [100, 10], 1), (3, [5, 1], 0),
     (2, [24, 24], 1), (2, [32, 32], 1), (2, [56, 10], 1), (2, [4, 200], 1),
     (2, [22, 23], 0), (2, [16, 16], 0), (2, [57, 9], 0), (2, [200, 4], 0),
     (1, [2, 2], 0), (1, [32, 32], 0), (1, [4, 250], 0),
