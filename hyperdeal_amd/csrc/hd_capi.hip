@@ -704,17 +704,22 @@ int hd_advection_create(hd_matrix_free *mf, const double *velocity,
           (faster(true, false) || faster(true, true) ||
            faster(false, false) || faster(false, true)))
         {
-          hd::CurvedHost hx, hv;
-          hd::curved_space_operator(mf->xmap, t, skew_factor, xc, xf, hx);
-          hd::curved_space_operator(mf->vmap, t, skew_factor, vc, vf, hv);
-          e = hd::curved_create(mf->dim_x, mf->dim_v, nd, hx, hv,
-                                &op->curved);
-          if (e != hipSuccess)
+          // (an operator without these tables takes the quadrature kernel)
+          try
             {
-              hd_advection_destroy(op);
-              return hip_fail(e, "hd_advection_create: cell matrices");
+              hd::CurvedHost hx, hv;
+              hd::curved_space_operator(mf->xmap, t, skew_factor, xc, xf, hx);
+              hd::curved_space_operator(mf->vmap, t, skew_factor, vc, vf, hv);
+              op->has_curved = hd::curved_create(mf->dim_x, mf->dim_v, nd, hx,
+                                                 hv, &op->curved) ==
+                               hipSuccess;
             }
-          op->has_curved = true;
+          catch (const std::bad_alloc &)
+            {
+              hd::curved_destroy(op->curved);
+            }
+          if (!op->has_curved)
+            (void)hipGetLastError();
         }
     }
   mf->n_ops += 1;
@@ -969,9 +974,15 @@ int hd_vlasov_poisson_create(hd_matrix_free *mf, double skew_factor,
       if (e == hipSuccess &&
           hd::vp_strips_supported(mf->dim_x, nd, op->xdev.n))
         {
-          e = hipMalloc(&op->strips, hd::vp_strips_bytes(nd, op->xdev.n));
-          if (e == hipSuccess)
+          // (without inboxes the solves run on one workgroup)
+          if (hipMalloc(&op->strips,
+                        hd::vp_strips_bytes(nd, op->xdev.n)) == hipSuccess)
             e = hd::vp_strips_reset(op->strips, nd, op->xdev.n);
+          else
+            {
+              op->strips = nullptr;
+              (void)hipGetLastError();
+            }
         }
     }
   if (e != hipSuccess)
