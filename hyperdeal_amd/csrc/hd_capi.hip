@@ -205,7 +205,7 @@ int run_operator(hd_advection *op, int mode, int precision, const void *src,
         return fail(HD_ERR_INVALID,
                     "the collapsed kernel needs a 16-byte aligned source "
                     "vector");
-      if (op->split && hd::collapsed_cres_supported(mf->D, mf->nd))
+      if (op->cres)
         e = precision == HD_FP64
               ? hd::collapsed_cres_f64(mf->nd, mode,
                                        static_cast<const double *>(src),
@@ -581,14 +581,15 @@ int hd_advection_create(hd_matrix_free *mf, const double *velocity,
   for (int d = 0; d < D; ++d)
     all_periodic = all_periodic && mf->periodic[d];
   op->dirichlet = !all_periodic;
-  op->split = !hd::collapsed_supported(D, nd) &&
-              hd::collapsed_split_supported(D, nd);
+  const bool lds = hd::collapsed_supported(D, nd);
+  op->cres = !lds && hd::collapsed_cres_supported(D, nd);
+  op->split = !lds && hd::collapsed_split_supported(D, nd);
   op->collapsed_ok =
     !mf->deformed &&
     (all_periodic ||
      hd::dirichlet_collapsed_supported(D, nq,
                                        bc_kind == HD_BC_INHOMOGENEOUS)) &&
-    (hd::collapsed_supported(D, nd) || op->split);
+    (lds || op->cres || op->split);
   if (op->collapsed_ok)
     {
       const int per = nd * nd + nd;
@@ -698,7 +699,7 @@ int hd_advection_create(hd_matrix_free *mf, const double *velocity,
         return hd::curved_faster(mf->dim_x, mf->dim_v, nd, mf->mesh.n_cells,
                                  fp64, stage);
       };
-      if (all_periodic &&
+      if (all_periodic && hd::quadrature_supported(D, nd, nq) &&
           hd::curved_supported(mf->dim_x, mf->dim_v, nd, mf->xmap.n_cells(),
                                mf->vmap.n_cells()) &&
           (faster(true, false) || faster(true, true) ||
@@ -1281,8 +1282,7 @@ int hd_lsrk_step(hd_advection *op, const char *type, int precision,
         sol, nullptr, op->vpdev, op->n_x_cells, op->n_v_cells, op->partial,
         op->density_chunks, op->rho, as_stream(stream),
         precision == HD_FP32 ? static_cast<float *>(ti_a) : nullptr,
-        precision == HD_FP64 && !from_sol ? static_cast<double *>(ti_a)
-                                          : nullptr);
+        precision == HD_FP64 ? static_cast<double *>(ti_a) : nullptr);
       rc = e == hipSuccess ? HD_OK : hip_fail(e, "hd_lsrk_step: density");
     }
   else if (!from_sol)

@@ -1341,7 +1341,7 @@ hipError_t split_launch(int mode, const T *src, T *dst, T *part,
                         const InflowDev &inflow, const StageDev &stage,
                         hipStream_t stream)
 {
-  static_assert(D == 5 || D == 6, "split form: D = 5, 6");
+  static_assert(D == 5, "split form");
   constexpr int R = D - 4;
   // 1) the slab view: a 4D mesh of n_cells * N^R slabs
   MeshDev m4 = mesh;
@@ -1412,7 +1412,7 @@ hipError_t split_dispatch(int D, int N, int mode, const T *src, T *dst,
 
 bool collapsed_split_supported(int D, int N)
 {
-  return (D == 5 || D == 6) && (N == 5 || N == 6);
+  return D == 5 && (N == 5 || N == 6);
 }
 
 hipError_t collapsed_split_f64(int D, int N, int mode, const double *src,

@@ -46,7 +46,8 @@ namespace hd
 namespace dirichlet
 {
 constexpr int kBlock = 256;
-// largest number of face quadrature points the collapsed path takes
+// Inhomogeneous data on more face points (3+3 with 7 or 8 points per direction)
+// is refused: no other kernel here takes those sizes, and none is tested there.
 constexpr int kMaxFacePoints = 7776;
 
 __host__ __device__ inline long long ipow_ll(int b, int e)

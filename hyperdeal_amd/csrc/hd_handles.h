@@ -150,7 +150,9 @@ struct hd_advection
   int algorithm = HD_ALGO_AUTO;
   bool collapsed_ok = false;
   bool dirichlet = false;      // some direction has Dirichlet boundaries
-  bool split = false;          // the collapsed form runs split (big cells)
+  // cells larger than LDS: the collapsed form runs in one pass from registers
+  // (6D) or split (5D)
+  bool cres = false, split = false;
   // a free vector (n_dofs doubles) for the last stage of the split form
   // (its first part) and of the FCL form (the assembled integrals)
   void *split_scratch = nullptr;

@@ -216,8 +216,8 @@ int hd_batch_size(const hd_batch *batch);
 int hd_batch_apply(hd_batch *batch, const void *const *src, void *const *dst,
                    int precision, void *stream);
 /* one LSRK step of every operator: sol[i] FP64, ti_a[i] != ti_b[i] stage
- * registers of `precision`; one copy launch and one launch per degree and
- * stage */
+ * registers of `precision`; one launch per degree and stage, after one copy
+ * launch in FP32 */
 int hd_batch_lsrk_step(hd_batch *batch, const char *type, int precision,
                        double *const *sol, void *const *ti_a,
                        void *const *ti_b, double dt, void *stream);
