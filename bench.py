@@ -382,7 +382,7 @@ def lsrk_precision_run(H, torch, stream, mf, op, u, vel, k, h):
 
 def c3_workload(H, torch, stream, steps):
     """3+3, k=5, 6^3 x 6^3 cells (46,656 DoF per cell, 2,176,782,336 DoF):
-    the split collapsed apply in FP64 and FP32-mixed, then 20 rk45 steps in
+    the one-pass collapsed apply in FP64 and FP32-mixed, then 20 rk45 steps in
     each precision from the same f0 (product of sines + 1e-3 noise, the C2
     seeds), dt = 0.1 * dt_crit / k^1.5.  Reported: apply GDoF/s and their
     ratio, the relative L2 difference FP32-mixed vs FP64 after 20 steps and
@@ -409,7 +409,7 @@ def c3_workload(H, torch, stream, steps):
     lsrk = lsrk_precision_run(H, torch, stream, mf, op, u, vel, k, 1.0 / 6)
     out = {
         "workload": "3D+3D apply, periodic [0,1]^6, 6^3 x 6^3 cells, k=5 "
-                    "(46656 DoF/cell, %d DoF), split collapsed form" % n,
+                    "(46656 DoF/cell, %d DoF), one-pass collapsed form" % n,
         "fp64": {"value": round(n / t64 / 1e9, 3), "unit": "GDoF/s",
                  "ms_per_apply": round(t64 * 1e3, 3),
                  "achieved_GBs": round(16.0 * n / t64 / 1e9, 1)},

@@ -3,7 +3,8 @@
 //
 // The collapsed operator (see hd_collapsed.hip) is a sum of 1D operators, one
 // per direction.  A block works on one cell at a time (k = 5 in FP64: two
-// blocks share a cell, every other output plane each); the cell's result
+// blocks share a cell, every other output plane each; few cells: a block per
+// plane); the cell's result
 // lives in the block's registers and the input streams through LDS one chunk
 // of fixed i5 (N^5 values) at a time:
 //   - thread t owns the chunk's values e = t + m BLOCK and the results

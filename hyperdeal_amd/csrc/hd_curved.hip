@@ -15,7 +15,7 @@
 // the host (curved_space_operator).  All x cells of a v cell share Kv, all v
 // cells of an x cell share Kx.
 //
-// Measured (2+2, k = 3, 24^4 cells, 85M values): FP64 apply 3218 -> 434 us
+// Measured (2+2, k = 3, 24^4 cells, 85M values): FP64 apply 3213 -> 434 us
 // (3.1 TB/s of its 16 bytes per value), FP32 2250 -> 200 us, against the
 // quadrature kernel; k = 4, 20^4 cells 4.1 -> 1.0 ms.
 //

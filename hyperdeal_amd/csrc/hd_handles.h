@@ -132,8 +132,9 @@ struct hd_learned_guess
   long long dense_solves = 0; // the first solves all train (then train_every)
   int train_every = 1, train_batch = 8, train_steps = 1, min_pairs = 4;
   float lr = 1e-3f;
-  // training runs on its own stream while the solve's CG (one workgroup)
-  // runs on the caller's: forked after the guess, joined before the next
+  // training runs on its own stream while the solve's CG (one workgroup, or
+  // up to 32) runs on the caller's: forked after the guess, joined before the
+  // next
   hipStream_t train_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_phi = nullptr, ev_done = nullptr;
   bool pending = false; // training enqueued and not yet joined

@@ -11,9 +11,10 @@
 //
 // The x-space problem is small (32^2 cells, 16,384 DoF at k=3), so the whole
 // solve runs in one workgroup (hd_vpcg.hip: in up to 32): every thread owns
-// whole x cells, the search direction lives in LDS (the SIPG face terms read the neighbour cells from
-// there), dot products are block reductions, and the iteration count stays
-// on the device -- no host round trip inside a Runge-Kutta stage.
+// whole x cells, the search direction lives in LDS (the SIPG face terms read
+// the neighbour cells from there), dot products are block reductions, and the
+// iteration count stays on the device -- no host round trip inside a
+// Runge-Kutta stage.
 #include "hd_device.h"
 #include "hd_vp_table.h"
 

@@ -5,7 +5,7 @@
 //
 // What bounds a solve is the latency of an iteration: on one workgroup a
 // matrix-vector product of 32^2 cells at k = 3 is 2,100 vector instructions
-// per wave on four SIMDs, 12 us per iteration.  Spread over 32 workgroups
+// per wave on four SIMDs, 11 us per iteration.  Spread over 32 workgroups
 // the product takes about 0.3 us and an iteration is one exchange between
 // workgroups.  Conjugate gradients in the form of Chronopoulos and Gear (1989)
 // needs a single reduction per iteration: with r known everywhere it is
@@ -34,9 +34,10 @@
 // the launch, whose work the small kernel launched behind this one then does
 // on its own; without the mark it returns at once.
 //
-// Measured (MI355X, k = 3): 12 -> 2.7 us per iteration at 32^2 x cells, 4.1 us
-// before the sums went through lane permutations and the stores that empty
-// slots overlapped the product; the check of an exact start 94 -> 12 us.
+// Measured (MI355X, k = 3, field updates of 393 iterations): 11.0 -> 3.1 us per
+// iteration at 32^2 x cells, 4.1 us before the sums went through lane
+// permutations and the stores that empty slots overlapped the product; the
+// check of an exact start 94 -> 12 us.
 #include "hd_device.h"
 
 #include <algorithm>
